@@ -166,16 +166,28 @@ def chain_launches(eng, dx, dy, batch, stream, reps=5):
     return statistics.median(a), statistics.median(e), ga, ge
 
 
+def sub_chains(cfg, batch):
+    """Parallel sub-chains of the engine's chain: two for a batch of more than
+    192 windows (MoE blocks) or 512 (dense)."""
+    windows = ((cfg.W + 7) // 8) * ((cfg.H + 7) // 8) * batch
+    return min(2, batch) if windows > (192 if cfg.n_experts > 1 else 512) else 1
+
+
+def w8(d, workgroups):
+    """The engine's attention runs as 8-wave workgroups for this many windows
+    (over a dense chain's sub-chains)."""
+    return "_w8" if workgroups < (257 if d == 256 else 512) else ""
+
+
 def expert_kernel(d, tokens, n_experts):
     """The expert kernel the engine's chain launches for `tokens` tokens: 128-
-    token tiles for d256 grids of >= 512 of them, else 64-token tiles (8 waves
-    below 512); grids hold ceil(tokens / tile) + one partial tile per expert,
-    rounded up to 8."""
+    token tiles for d256 grids of >= 512 of them, else 64-token tiles; grids
+    hold ceil(tokens / tile) + one partial tile per expert, rounded up to 8."""
     part = n_experts if n_experts > 1 else 0
     tiles = lambda bm: ((tokens + bm - 1) // bm + part + 7) // 8 * 8
     if d == 256 and tiles(128) >= 512:
         return f"prism_expert_d{d}_bm128"
-    return f"prism_expert_d{d}_bm64" + ("_w8" if tiles(64) < 512 else "")
+    return f"prism_expert_d{d}_bm64" + ("_w8" if tiles(64) < (321 if d == 256 else 512) else "")
 
 
 def measured_traffic(kernel, grid):
@@ -282,14 +294,14 @@ def config_section(hip, name, batch, steps, stream):
     finally:
         eng.close()
     flops_frame = cfg.flops_per_token_block() * T * cfg.n_blocks
-    S = max(1, min(2, batch // 2))  # the engine's sub-chains (CHAIN_SPLIT = 2 of >= 2 frames)
+    S = sub_chains(cfg, batch)
     tok_launch = batch * T // S
     a_flops = (attn_flops_per_token(cfg) + router_flops_per_token(cfg)) * tok_launch
     e_flops = 2 * 2 * d * d * tok_launch
     fused = ge == 0  # dense d128 blocks: the FFN runs inside the attention launch
     if fused:
         a_flops += e_flops
-    kern = f"prism_attn_d{d}" + ("_w8" if ga < 512 else "") + (f"_r{(cfg.n_experts + 15) // 16}" if cfg.n_experts > 1 else "") + ("_ffn" if fused else "")
+    kern = f"prism_attn_d{d}" + w8(d, ga if cfg.n_experts > 1 else ga * S) + (f"_r{(cfg.n_experts + 15) // 16}" if cfg.n_experts > 1 else "") + ("_ffn" if fused else "")
     return {"batch": batch, "ms_per_step": round(ms_b, 5), "frames_per_s": round(batch / (ms_b * 1e-3), 2),
             "mfma_frac": round(flops_frame * batch / (ms_b * 1e-3) / MFMA_F16_PEAK, 4),
             "batch1_us_per_frame": round(ms_1 * 1e3, 2),
@@ -366,7 +378,7 @@ def main():
     log("[bench] per-stage timing")
     t_attn = time_stage(hip, lambda: eng.attn(a_push, feats, B, stream), args.stage_reps, stream)
     attn_grid = ((cfg.W + 7) // 8) * ((cfg.H + 7) // 8) * B
-    kname = f"prism_attn_d{d}" + ("_w8" if attn_grid < 512 else "")
+    kname = f"prism_attn_d{d}" + w8(d, attn_grid)
     if moe:
         r_push = eng.router_push(0, T, n * d, 0, n, n + N)
         e_push = eng.expert_push(0, T, n * d, 0, 0, n, n + N)
@@ -395,14 +407,14 @@ def main():
     # one after another with HIP events between them
     log("[bench] chain launches")
     c_attn, c_exp, c_ga, c_ge = chain_launches(eng, dx, dy, B, stream)
-    S = max(1, min(2, B // 2))  # sub-chains of the engine (CHAIN_SPLIT = 2 of >= 2 frames)
+    S = sub_chains(cfg, B)
     tok_launch = n // S
     c_attn_flops = (attn_flops_per_token(cfg) + router_flops_per_token(cfg)) * tok_launch
     c_exp_flops = 2 * 2 * d * d * tok_launch
     c_fused = c_ge == 0  # dense d128 blocks: the FFN runs inside the attention launch
     if c_fused:
         c_attn_flops, c_exp_flops = c_attn_flops + c_exp_flops, 0
-    c_kname = (f"prism_attn_d{d}" + ("_w8" if c_ga < 512 else "") + (f"_r{(N + 15) // 16}" if moe else "")
+    c_kname = (f"prism_attn_d{d}" + w8(d, c_ga if moe else c_ga * S) + (f"_r{(N + 15) // 16}" if moe else "")
                + ("_ffn" if c_fused else ""))
     c_ename = None if c_fused else expert_kernel(d, tok_launch, N)
     c_traffic, c_traffic_src = measured_traffic(c_kname, c_ga) if cfg.name == "moe64" else (None, None)

@@ -37,17 +37,21 @@ using prism::DevBlock;
  * routed attention launch adds to them, and counters sharing a cache line
  * would serialise those atomics in one memory channel. */
 static constexpr int CHAIN_COUNT_STRIDE = 64;
-/* The chain runs as up to CHAIN_SPLIT independent sub-chains, one per
- * CHAIN_SPLIT_FRAMES frames, on their own streams (parallel branches of the
- * hipGraph): windows and tokens never interact across frames, and one
- * sub-chain's expert launches overlap another's attention launches and the
- * tails of both. */
+/* Compute units of an MI355X. */
+static constexpr int CU_COUNT = 256;
+/* The chain of a batch with more than CHAIN_SPLIT_ROUTED (MoE blocks) or
+ * CHAIN_SPLIT_DENSE windows (see chain_split) runs as up to CHAIN_SPLIT
+ * independent sub-chains of whole frames, on their own streams
+ * (parallel branches of the hipGraph): windows and tokens never interact
+ * across frames, and one sub-chain's expert launches overlap another's
+ * attention launches and the tails of both. */
 static constexpr int CHAIN_SPLIT = 2;
-static constexpr int CHAIN_SPLIT_FRAMES = 2;
+static constexpr int CHAIN_SPLIT_ROUTED = CU_COUNT * 3 / 4;
+static constexpr int CHAIN_SPLIT_DENSE = 2 * CU_COUNT;
 static_assert(CHAIN_SPLIT >= 1 && CHAIN_SPLIT <= 4, "sub-chain streams");
 /* d256 expert launches of at least this many 128-token tiles (two per CU)
  * use the 128-token kernel: each streamed weight fragment then feeds twice
- * the tokens. Smaller grids keep 64-token tiles (8 waves below 512 tiles).
+ * the tokens. Smaller grids keep 64-token tiles (8 waves up to CU_COUNT tiles).
  * A stage call of that size uses 96-token tiles of the same body instead:
  * alone on the GPU, its last round of workgroups is then less empty (batch 8
  * to 16 at 68x120: 7-13 % faster); inside the block chain the other
@@ -55,8 +59,8 @@ static_assert(CHAIN_SPLIT >= 1 && CHAIN_SPLIT <= 4, "sub-chain streams");
  * ahead there. */
 static constexpr int EXPERT_WIDE_MIN_TILES = 512;
 /* The share of the 256 MB memory-side cache the weights may keep across
- * small-batch frames: when a model's weights exceed it, the 8-wave 64-token
- * expert kernel (the small grids of batch 1-2) reads the expert weights of
+ * small-batch frames: when a model's weights exceed it, the d256 64-token
+ * expert kernels (the grids of a few frames) read the expert weights of
  * the first blocks non-temporally, so the rest stays resident from one frame
  * to the next instead of the whole cyclic stream missing (prism_load_weights
  * sets wnt_blocks). */

@@ -482,10 +482,12 @@ struct RouteOut {
     int32_t* zero_next; /* counters this launch clears for a later one, or NULL */
 };
 
-/* ffn: a dense block's FFN runs in the same launch (the window's rows never
+/* par: attention launches of about this size that run at the same time (a
+ * dense chain's sub-chains; a routed one's run beside the other's experts).
+ * ffn: a dense block's FFN runs in the same launch (the window's rows never
  * leave the CU between the two), and `out` receives the block's output */
 int enqueue_attn(prism_ctx* c, const DevBlock& k, const uint16_t* in, uint16_t* out, int H, int W, int batch,
-                 hipStream_t s, const RouteOut* route = nullptr, bool up = false, bool ffn = false) {
+                 hipStream_t s, const RouteOut* route = nullptr, bool up = false, bool ffn = false, int par = 1) {
     const int D = c->desc.dim;
     if (ffn && (route || c->desc.n_experts != 1))
         return fail(c, PRISM_ERR_INVALID, "the fused FFN is for dense blocks");
@@ -529,9 +531,16 @@ int enqueue_attn(prism_ctx* c, const DevBlock& k, const uint16_t* in, uint16_t* 
     }
     const int64_t grid = (int64_t)a.windows_per_frame * batch;
     if (grid <= 0 || grid > 0x7fffffff) return fail(c, PRISM_ERR_INVALID, "attention grid %lld out of range", (long long)grid);
-    /* fewer than two windows per CU: one 8-wave workgroup per window (a head per
-     * wave) shortens each window's serial path; otherwise 4 waves x 2 per CU */
-    const int w8 = grid < 512 ? 1 : 0;
+    /* Windows that fit the CUs as 8-wave workgroups (a head per wave) take
+     * those, which shortens each window's serial path; more of them go as
+     * 4-wave workgroups, two per CU (three at d128). A d256 8-wave workgroup fills its CU's registers,
+     * so window 257 starts a second round: routed launches of 270, 405 and
+     * 510 windows take 28.6, 32.6 and 35 us on 8 waves, 23.6, 27.5 and 30.7
+     * on 4, and one of 135 takes 16.8 us on 8. Two d128 ones share a CU (270
+     * windows 13.0 us either way, 405 16.3 and 16.0). With par > 1 the
+     * launches' windows count together (two dense launches of 256 at once: 162
+     * us a four-block chain on 8 waves, 134 on 4). */
+    const int w8 = grid * par < (D == 256 ? CU_COUNT + 1 : 2 * CU_COUNT) ? 1 : 0;
     const hipFunction_t f = ffn ? c->f_attn_ffn[dim_index(D)][w8] : c->f_attn[dim_index(D)][w8][npt];
     if (!f) return fail(c, PRISM_ERR_INVALID, "no fused FFN kernel for d%d at %lld windows", D, (long long)grid);
     return launch(c, f, (unsigned)grid, a, s, w8 ? 512u : 256u);
@@ -597,8 +606,16 @@ int enqueue_experts(prism_ctx* c, const DevBlock& k, const uint16_t* in, uint16_
         return stage ? launch(c, c->f_expert_wide96, (unsigned)tiles_of(96), a, s, 256u)
                      : launch(c, c->f_expert_wide, (unsigned)tiles_of(128), a, s, 256u);
     const int64_t tiles = tiles_of(64);
-    /* fewer tiles than two per CU: 8 waves per tile halve each wave's weight stream */
-    const int w8 = tiles < 512 ? 1 : 0;
+    /* at most one tile per CU: 8 waves per tile halve each wave's weight
+     * stream; otherwise 4 waves x 2 tiles per CU. 64 experts alone on the GPU,
+     * 320 and 448 tiles: 20.9 and 21.7 us on 8 waves (a round of 256 and one
+     * of the rest), 18.6 and 19.6 us on 4. Beside the other sub-chain's
+     * attention a small second round costs less than slower tiles: a chain
+     * with launches of 280 tiles 696 us on 8 waves, 770 on 4; of 296, 745 and
+     * 789; of 320, 816 and 832 (or 807 and 789); of 352, 891 and 855. d128
+     * tiles leave room for two 8-wave workgroups per CU. */
+    const int64_t w8_tiles = D == 256 ? (stage ? CU_COUNT : CU_COUNT * 5 / 4) : 2 * CU_COUNT - 1;
+    const int w8 = tiles <= w8_tiles ? 1 : 0;
     return launch(c, c->f_expert[dim_index(D)][w8], (unsigned)tiles, a, s, w8 ? 512u : 256u);
 }
 
@@ -883,8 +900,24 @@ static int ensure_workspace(prism_ctx* c, int batch, bool io = false) {
  * chain leaves row 0 at zero. The workspace starts zeroed; a one-block model
  * clears its row inside the chain; after a chain that failed part-way, the
  * next prism_forward / prism_forward_graph call clears the counters first.
- * With 2 * CHAIN_SPLIT_FRAMES frames or more the batch runs as sub-chains
- * (own counter rows, own bucket region, disjoint frames of every buffer). */
+ * A large batch runs as sub-chains (own counter rows, own bucket region,
+ * disjoint frames of every buffer). */
+
+/* Sub-chains of a forward. A routed block's two launches leave CUs idle in
+ * turn (the attention's while its last windows finish, the experts' while
+ * they wait for weights), so the frames of a batch go in halves as soon as
+ * one half's attention launch no longer fits beside the other's experts for
+ * free: 16 blocks, one chain against two: 160 windows 411 and 418 us, 192
+ * 442 and 438, 256 578 and 509 (64 experts), 270 641 and 504, 288 684 and
+ * 539, 504 859 and 814. A dense block is one launch: its frames stay together
+ * while they fit one round of the 4-wave kernels (two workgroups per CU; four
+ * blocks, 256 windows 83 and 91 us, d128 512 windows 61 and 74; 540 windows
+ * 170 and 150). */
+static int chain_split(const prism_model_desc& d, int batch) {
+    const int64_t windows = (int64_t)((d.spatial_w + 7) / 8) * ((d.spatial_h + 7) / 8) * batch;
+    return windows > (d.n_experts > 1 ? CHAIN_SPLIT_ROUTED : CHAIN_SPLIT_DENSE) ? std::min(CHAIN_SPLIT, batch) : 1;
+}
+
 /* Sub-chain j: frames [f0, f0 + nf) through every block, in -> out (this
  * sub-chain's frames). adapted: in and out hold 128-channel rows; block 0's
  * attention runs the up-projection in its prologue and the last block's
@@ -912,7 +945,7 @@ static int timer_mark(prism_ctx* c, ChainTimer* tm, int kind, hipStream_t s) {
     return PRISM_OK;
 }
 
-static int enqueue_subchain(prism_ctx* c, const ChainWs& ws, int j, int f0, int nf, const uint16_t* in,
+static int enqueue_subchain(prism_ctx* c, const ChainWs& ws, int S, int j, int f0, int nf, const uint16_t* in,
                             uint16_t* out, hipStream_t s, bool adapted = false, ChainTimer* tm = nullptr) {
     const int NB = c->desc.n_blocks, H = c->desc.spatial_h, W = c->desc.spatial_w, D = c->desc.dim;
     const int N = c->desc.n_experts;
@@ -945,11 +978,11 @@ static int enqueue_subchain(prism_ctx* c, const ChainWs& ws, int j, int f0, int 
             if (!rc) rc = timer_mark(c, tm, 1, s);
             if (rc) return rc;
         } else if (!last) { /* one launch: attention + the FFN */
-            int rc = enqueue_attn(c, k, src, dst, H, W, nf, s, nullptr, first, true);
+            int rc = enqueue_attn(c, k, src, dst, H, W, nf, s, nullptr, first, true, S);
             if (!rc) rc = timer_mark(c, tm, 0, s);
             if (rc) return rc;
         } else {
-            int rc = enqueue_attn(c, k, src, attn, H, W, nf, s, nullptr, first);
+            int rc = enqueue_attn(c, k, src, attn, H, W, nf, s, nullptr, first, false, S);
             if (!rc) rc = timer_mark(c, tm, 0, s);
             if (!rc) rc = enqueue_experts(c, k, attn, dst, nullptr, nullptr, n, s, 1, last);
             if (!rc) rc = timer_mark(c, tm, 1, s);
@@ -966,8 +999,8 @@ static int enqueue_forward_impl(prism_ctx* c, const ChainWs& ws, const uint16_t*
     const int64_t D = adapted ? c->aoffs.in_dim : c->desc.dim; /* channels of in and out */
     c->fwd_tokens = (int64_t)batch * T;
     c->fwd_assign = ws.assign;
-    const int S = std::max(1, std::min(CHAIN_SPLIT, batch / CHAIN_SPLIT_FRAMES));
-    if (S == 1) return enqueue_subchain(c, ws, 0, 0, batch, in, out, s, adapted);
+    const int S = chain_split(c->desc, batch);
+    if (S == 1) return enqueue_subchain(c, ws, 1, 0, 0, batch, in, out, s, adapted);
     /* fork: sub-chain j > 0 on sub_stream[j-1], sub-chain 0 on s, then join */
     HIP_TRY(c, hipEventRecord(c->ev_fork, s));
     int rc = PRISM_OK;
@@ -975,7 +1008,7 @@ static int enqueue_forward_impl(prism_ctx* c, const ChainWs& ws, const uint16_t*
         const int f0 = (int)((int64_t)batch * j / S), f1 = (int)((int64_t)batch * (j + 1) / S);
         hipStream_t sj = j ? c->sub_stream[j - 1] : s;
         if (j) HIP_TRY(c, hipStreamWaitEvent(sj, c->ev_fork, 0));
-        const int r = enqueue_subchain(c, ws, j, f0, f1 - f0, in + f0 * T * D, out + f0 * T * D, sj, adapted);
+        const int r = enqueue_subchain(c, ws, S, j, f0, f1 - f0, in + f0 * T * D, out + f0 * T * D, sj, adapted);
         if (!rc) rc = r;
         if (j) HIP_TRY(c, hipEventRecord(c->ev_join[j - 1], sj));
     }
@@ -1132,7 +1165,7 @@ extern "C" int prism_chain_launch_times(prism_ctx* c, const void* in, void* out,
     c->fwd_tokens = ws.n;
     c->fwd_assign = ws.assign;
     /* the sub-chains of prism_forward, one after another on one stream */
-    const int S = std::max(1, std::min(CHAIN_SPLIT, batch / CHAIN_SPLIT_FRAMES));
+    const int S = chain_split(c->desc, batch);
     ChainTimer tm;
     tm.ev.assign((size_t)2 * c->desc.n_blocks * S + 1, nullptr);
     for (auto& e : tm.ev) {
@@ -1148,7 +1181,7 @@ extern "C" int prism_chain_launch_times(prism_ctx* c, const void* in, void* out,
     rc = timer_mark(c, &tm, -1, s);
     for (int j = 0; j < S && !rc; ++j) {
         const int f0 = (int)((int64_t)batch * j / S), f1 = (int)((int64_t)batch * (j + 1) / S);
-        rc = enqueue_subchain(c, ws, j, f0, f1 - f0, src + f0 * T * D, dst + f0 * T * D, s, false, &tm);
+        rc = enqueue_subchain(c, ws, S, j, f0, f1 - f0, src + f0 * T * D, dst + f0 * T * D, s, false, &tm);
     }
     if (rc) c->counts_dirty = true; /* launched part of the chain */
     double sum[2] = {0, 0};

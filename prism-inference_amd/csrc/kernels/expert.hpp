@@ -134,8 +134,18 @@ __device__ __forceinline__ void expert_stage_tile(const ExpertArgs& a, int e, in
     if (i < BM) tok[i] = t;
 }
 
+/* The workgroup's LDS, declared once per kernel: both instantiations of the
+ * body (weights read through the caches or past them) use the same arrays. */
+template <int DIM, int BM>
+struct ExpertLds {
+    __attribute__((aligned(16))) f16 xs[BM * (DIM + 8)]; /* LN2 output, then GELU output */
+    __attribute__((aligned(16))) f16 hs[BM * (DIM + 8)]; /* raw rows (residual)          */
+    float b1[DIM], b2[DIM];
+    int tok[BM];
+};
+
 template <int DIM, int BM, int NW, bool WNT = false>
-__device__ __forceinline__ void expert_body(const ExpertArgs& a) {
+__device__ __forceinline__ void expert_body(const ExpertArgs& a, ExpertLds<DIM, BM>& L) {
     constexpr int WP = WNT ? 2 : 0; /* weight loads' cache policy */
     static_assert(NW == 4 || NW == 8, "4 or 8 waves");
     constexpr int NT = 64 * NW;   /* threads                          */
@@ -147,10 +157,11 @@ __device__ __forceinline__ void expert_body(const ExpertArgs& a) {
     constexpr int RPI = 64 / LPS; /* LN rows per wave iteration       */
     static_assert(RT >= 1 && BM % (NW * RPI) == 0, "tile shape");
 
-    __shared__ __attribute__((aligned(16))) f16 xs[BM * LDS]; /* LN2 output, then GELU output */
-    __shared__ __attribute__((aligned(16))) f16 hs[BM * LDS]; /* raw rows (residual)          */
-    __shared__ float s_b1[DIM], s_b2[DIM];
-    __shared__ int tok[BM];
+    f16* const xs = L.xs;
+    f16* const hs = L.hs;
+    float* const s_b1 = L.b1;
+    float* const s_b2 = L.b2;
+    int* const tok = L.tok;
 
     const int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -568,19 +579,26 @@ __device__ __forceinline__ void expert_wide(const ExpertArgs& a, ExpertWideLds<D
 /* 4 waves (2 workgroups per CU) for large grids; 8 waves (each streaming half
  * as many weight rows) when tiles are scarcer than CUs. */
 extern "C" __global__ void __launch_bounds__(256, 2) prism_expert_d256_bm64(ExpertArgs a) {
-    expert_body<256, 64, 4>(a);
+    __shared__ ExpertLds<256, 64> lds;
+    if (a.wnt) /* uniform */
+        expert_body<256, 64, 4, true>(a, lds);
+    else
+        expert_body<256, 64, 4>(a, lds);
 }
 extern "C" __global__ void __launch_bounds__(256, 2) prism_expert_d128_bm64(ExpertArgs a) {
-    expert_body<128, 64, 4>(a);
+    __shared__ ExpertLds<128, 64> lds;
+    expert_body<128, 64, 4>(a, lds);
 }
 extern "C" __global__ void __launch_bounds__(512, 1) prism_expert_d256_bm64_w8(ExpertArgs a) {
+    __shared__ ExpertLds<256, 64> lds;
     if (a.wnt) /* uniform */
-        expert_body<256, 64, 8, true>(a);
+        expert_body<256, 64, 8, true>(a, lds);
     else
-        expert_body<256, 64, 8>(a);
+        expert_body<256, 64, 8>(a, lds);
 }
 extern "C" __global__ void __launch_bounds__(512, 1) prism_expert_d128_bm64_w8(ExpertArgs a) {
-    expert_body<128, 64, 8>(a);
+    __shared__ ExpertLds<128, 64> lds;
+    expert_body<128, 64, 8>(a, lds);
 }
 /* 128-token tiles, 4 waves, 2 workgroups per CU: the large grids of batched
  * launches (no fused down-projection) */
