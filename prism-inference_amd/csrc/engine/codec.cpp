@@ -6,12 +6,13 @@
  * Weights arrive in the reference's layouts (row-major [out][in]; conv
  * columns k = ic*9 + ky*3 + kx) and are repacked once into MFMA A-fragment
  * order: the stride-2 convs with columns reordered to k = tap*Cin + ic (the
- * kernels read NHWC taps), the input conv with its 81 columns as 9 taps x 16,
+ * kernels read NHWC taps), the input conv with its 81 columns as 3 kernel rows of 3 x 10 (+ 2),
  * the output conv with rows padded to 16 and columns permuted to the
  * accumulator-lane order its fused kernel feeds it in. Biases become fp32.
  */
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -24,15 +25,16 @@ using namespace prism;
 namespace {
 
 enum { ST_ENC0, ST_ENC1, ST_ENC2, ST_ENC3, ST_DEC3, ST_DEC2, ST_DEC1, N_STAGES };
-const int kTT[N_STAGES] = {4, CODEC_TT_ENC1, CODEC_TT_ENC2, CODEC_TT_ENC3, /* enc0: own grid */
-                           CODEC_TT_DEC3, CODEC_TT_DEC2, CODEC_TT_DEC1};
-const int kRS[N_STAGES] = {1, CODEC_RS_ENC1, CODEC_RS_ENC2, CODEC_RS_ENC3, CODEC_RS_DEC3, CODEC_RS_DEC2, 1};
-const int kKSP[N_STAGES] = {1, CODEC_KSP_ENC1, CODEC_KSP_ENC2, CODEC_KSP_ENC3, CODEC_KSP_DEC3, CODEC_KSP_DEC2, 1};
+const int kTT[N_STAGES] = {0, CODEC_TT_ENC1, 0, 0, 0, CODEC_TT_DEC2, CODEC_TT_DEC1}; /* 0: a grid of its own */
 const int kInRes[N_STAGES] = {0, 0, 1, 2, 3, 2, 1};  /* resolution index of the (coarse) input map */
 const int kOutRes[N_STAGES] = {0, 1, 2, 3, 2, 1, 0}; /* of the output map (dec1: before the shuffle) */
 const int kInCh[N_STAGES] = {9, 32, 64, 128, 128, 128, 64};
 const int kSkipCh[N_STAGES] = {0, 0, 0, 0, 128, 64, 32};
 const int kOutCh[N_STAGES] = {32, 64, 128, 128, 128, 64, 12}; /* dec1: 12 channels = 3 planes x 2x2 */
+
+/* workgroups of the persistent codec launches the GPU holds at once */
+constexpr int CODEC_DEC3_SLOTS = 3 * CU_COUNT, CODEC_DEC21_SLOTS = 3 * CU_COUNT, CODEC_ENC01_SLOTS = 2 * CU_COUNT,
+              CODEC_ENC2_SLOTS = 2 * CU_COUNT, CODEC_ENC3_SLOTS = 2 * CU_COUNT;
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
@@ -61,34 +63,64 @@ CodecArgs stage_args(const prism_ctx* c, int st, const uint16_t* in, const uint1
     return a;
 }
 
+/* Grid of a persistent decoder launch: `slots` workgroups at once, every one
+ * the same number of the launch's blocks (or one fewer), so no workgroup is
+ * left with a block of its own at the end. */
+unsigned even_grid(int64_t blocks, int slots) {
+    const int64_t each = (blocks + slots - 1) / slots;
+    return (unsigned)((blocks + each - 1) / each);
+}
+
+/* Blocks of rows x cols pixels of a w x h map. */
+int blocks_of(int w, int h, int rows, int cols) { return ((w + cols - 1) / cols) * ((h + rows - 1) / rows); }
+
+/* Launches a persistent kernel over `per_frame` blocks of each frame; its last
+ * two arguments are the block counts. xcd: the grid is a whole number of turns
+ * over the XCDs, so a workgroup's blocks stay in its XCD's band. */
+template <class... A>
+int launch_blocks(prism_ctx* c, hipFunction_t f, const char* what, int per_frame, int batch, int slots, bool xcd,
+                  unsigned threads, hipStream_t s, A&... args) {
+    const int64_t blocks = (int64_t)per_frame * batch;
+    if (blocks > INT32_MAX / 2) return fail(c, PRISM_ERR_INVALID, "%s: %lld blocks", what, (long long)blocks);
+    int nblk = (int)blocks;
+    unsigned grid = even_grid(blocks, slots);
+    if (xcd) grid = (grid + 7) / 8 * 8;
+    void* params[] = {&args..., &per_frame, &nblk};
+    const hipError_t e = hipModuleLaunchKernel(f, grid, 1, 1, threads, 1, 1, 0, s, params, nullptr);
+    if (e != hipSuccess) return fail(c, PRISM_ERR_HIP, "hipModuleLaunchKernel(%s): %s", what, hipGetErrorString(e));
+    return PRISM_OK;
+}
+
 int launch_stage(prism_ctx* c, int st, const uint16_t* in, const uint16_t* skip, uint16_t* out, int batch,
                  hipStream_t s) {
     CodecArgs a = stage_args(c, st, in, skip, out);
+    if (st == ST_ENC2)
+        return launch_blocks(c, c->f_codec[st], "enc2", blocks_of(a.out_w, a.out_h, CODEC_ENC2_ROWS, CODEC_ENC2_COLS), batch,
+                             CODEC_ENC2_SLOTS, true, 512, s, a);
+    if (st == ST_ENC3)
+        return launch_blocks(c, c->f_codec[st], "enc3", blocks_of(a.out_w, a.out_h, CODEC_ENC3_ROWS, CODEC_ENC3_COLS), batch,
+                             CODEC_ENC3_SLOTS, true, 512, s, a);
+    if (st == ST_DEC3)
+        return launch_blocks(c, c->f_codec[st], "dec3", blocks_of(a.out_w, a.out_h, CODEC_DEC_ROWS, CODEC_DEC_COLS), batch,
+                             CODEC_DEC3_SLOTS, false, 256, s, a);
     const int64_t out_pix = (int64_t)a.out_w * a.out_h;
-    const int64_t per_wg = 64 * kTT[st] / (kRS[st] * kKSP[st]); /* pixels per workgroup */
-    const unsigned gx = st == ST_ENC0 ? (unsigned)(((a.out_w + CODEC_ENC0_COLS - 1) / CODEC_ENC0_COLS) *
-                                                  ((a.out_h + CODEC_ENC0_ROWS - 1) / CODEC_ENC0_ROWS))
-                        : st == ST_ENC2 ? (unsigned)(((a.out_w + CODEC_WIN_COLS_ENC2 - 1) / CODEC_WIN_COLS_ENC2) *
-                                                     ((a.out_h + CODEC_WIN_ROWS_ENC2 - 1) / CODEC_WIN_ROWS_ENC2))
-                                        : (unsigned)((out_pix + per_wg - 1) / per_wg);
+    const int64_t per_wg = 64 * kTT[st]; /* pixels per workgroup */
+    const unsigned gx = st == ST_ENC0 ? (unsigned)blocks_of(a.out_w, a.out_h, CODEC_ENC0_ROWS, CODEC_ENC0_COLS)
+                                      : (unsigned)((out_pix + per_wg - 1) / per_wg);
     void* params[] = {&a};
     const hipError_t e = hipModuleLaunchKernel(c->f_codec[st], gx, (unsigned)batch, 1, 256, 1, 1, 0, s, params, nullptr);
     if (e != hipSuccess) return fail(c, PRISM_ERR_HIP, "hipModuleLaunchKernel(codec stage %d): %s", st, hipGetErrorString(e));
     return PRISM_OK;
 }
 
-/* dec2 and dec1_out as one launch (prism_codec_dec21_out): 2 x 32 blocks of
- * the r1 map, each with the 4 x 64 r0 block above it. d2 = the dec3 map, e1
- * and e0 the skips. */
+/* dec2 and dec1_out as one launch (prism_codec_dec21_out). d3 = the dec3 map,
+ * e1 and e0 the skips. */
 int launch_dec21(prism_ctx* c, const uint16_t* d3, const uint16_t* e1, const uint16_t* e0, uint16_t* display,
                  int batch, hipStream_t s) {
     CodecArgs a2 = stage_args(c, ST_DEC2, d3, e1, nullptr);
     CodecArgs a1 = stage_args(c, ST_DEC1, nullptr, e0, display);
-    const unsigned gx = (unsigned)(((a2.out_w + 31) / 32) * ((a2.out_h + 1) / 2));
-    void* params[] = {&a2, &a1};
-    const hipError_t e = hipModuleLaunchKernel(c->f_codec21, gx, (unsigned)batch, 1, 256, 1, 1, 0, s, params, nullptr);
-    if (e != hipSuccess) return fail(c, PRISM_ERR_HIP, "hipModuleLaunchKernel(dec2 + dec1): %s", hipGetErrorString(e));
-    return PRISM_OK;
+    return launch_blocks(c, c->f_codec21, "dec2 + dec1", blocks_of(a2.out_w, a2.out_h, CODEC_DEC_ROWS, CODEC_DEC_COLS), batch,
+                         CODEC_DEC21_SLOTS, false, 256, s, a2, a1);
 }
 
 /* Packed copy of W[rows][K] with column j of the packed matrix taken from
@@ -163,37 +195,18 @@ int codec_ensure_workspace(prism_ctx* c, int batch) {
     return PRISM_OK;
 }
 
-/* enc0 and enc1 as one launch (prism_codec_enc01): CODEC_ENC01_ROWS x
- * CODEC_ENC01_COLS blocks of the r1 map, each with the e0 region under it;
- * writes both maps. */
+/* enc0 and enc1 as one launch (prism_codec_enc01), writing both maps. */
 int launch_enc01(prism_ctx* c, const uint16_t* frame, uint16_t* e0, uint16_t* e1, int batch, hipStream_t s) {
     CodecArgs a0 = stage_args(c, ST_ENC0, frame, nullptr, e0);
     CodecArgs a1 = stage_args(c, ST_ENC1, nullptr, nullptr, e1);
-    const unsigned gx = (unsigned)(((a1.out_w + CODEC_ENC01_COLS - 1) / CODEC_ENC01_COLS) *
-                                   ((a1.out_h + CODEC_ENC01_ROWS - 1) / CODEC_ENC01_ROWS));
-    void* params[] = {&a0, &a1};
-    const hipError_t e = hipModuleLaunchKernel(c->f_enc01, gx, (unsigned)batch, 1, 256, 1, 1, 0, s, params, nullptr);
-    if (e != hipSuccess) return fail(c, PRISM_ERR_HIP, "hipModuleLaunchKernel(enc0 + enc1): %s", hipGetErrorString(e));
-    return PRISM_OK;
-}
-
-/* enc2 and enc3 as one launch (prism_codec_enc23): CODEC_ENC23_ROWS x
- * CODEC_ENC23_COLS blocks of the bottleneck, each with the e2 region and the
- * e1 window under it; writes the e2 map and the bottleneck. 8 waves. */
-int launch_enc23(prism_ctx* c, const uint16_t* e1, uint16_t* e2, uint16_t* bottleneck, int batch, hipStream_t s) {
-    CodecArgs a2 = stage_args(c, ST_ENC2, e1, nullptr, e2);
-    CodecArgs a3 = stage_args(c, ST_ENC3, nullptr, nullptr, bottleneck);
-    const unsigned gx = (unsigned)(((a3.out_w + CODEC_ENC23_COLS - 1) / CODEC_ENC23_COLS) *
-                                   ((a3.out_h + CODEC_ENC23_ROWS - 1) / CODEC_ENC23_ROWS));
-    void* params[] = {&a2, &a3};
-    const hipError_t e = hipModuleLaunchKernel(c->f_enc23, gx, (unsigned)batch, 1, 512, 1, 1, 0, s, params, nullptr);
-    if (e != hipSuccess) return fail(c, PRISM_ERR_HIP, "hipModuleLaunchKernel(enc2 + enc3): %s", hipGetErrorString(e));
-    return PRISM_OK;
+    return launch_blocks(c, c->f_enc01, "enc0 + enc1", blocks_of(a1.out_w, a1.out_h, CODEC_ENC01_ROWS, CODEC_ENC01_COLS),
+                         batch, CODEC_ENC01_SLOTS, true, 512, s, a0, a1);
 }
 
 int codec_enqueue_encode(prism_ctx* c, const uint16_t* frame, uint16_t* bottleneck, int batch, hipStream_t s) {
     int rc = launch_enc01(c, frame, c->ce0, c->ce1, batch, s);
-    if (!rc) rc = launch_enc23(c, c->ce1, c->ce2, bottleneck, batch, s);
+    if (!rc) rc = launch_stage(c, ST_ENC2, c->ce1, nullptr, c->ce2, batch, s);
+    if (!rc) rc = launch_stage(c, ST_ENC3, c->ce2, nullptr, bottleneck, batch, s);
     return rc;
 }
 
@@ -216,10 +229,13 @@ extern "C" int prism_load_codec(prism_ctx* c, const void* blob, size_t bytes, co
 
     std::vector<uint16_t> packed[8];
     const auto id = [](int j) { return j; };
-    /* enc0: packed column tap*16 + ic (9 taps x 16, 160 columns; ic >= 9 and
-     * tap 9 are zero) <- stored column ic*9 + tap */
-    pack_mapped(w + o->enc0_w, 32, 81, 32, 160,
-                [](int j) { const int tap = j / 16, ic = j % 16; return tap < 9 && ic < 9 ? ic * 9 + tap : -1; },
+    /* enc0: packed column 32 ky + 10 kx + ic (3 k-steps, the rest zero) <-
+     * stored column ic*9 + 3 ky + kx */
+    pack_mapped(w + o->enc0_w, 32, 81, 32, 96,
+                [](int j) {
+                    const int ky = j / 32, kx = j % 32 / 10, ic = j % 32 % 10;
+                    return kx < 3 && ic < 9 ? ic * 9 + 3 * ky + kx : -1;
+                },
                 packed[0]);
     /* enc1..3: packed column tap*Cin + ic <- stored column ic*9 + tap */
     const int cins[3] = {32, 64, 128}, couts[3] = {64, 128, 128};

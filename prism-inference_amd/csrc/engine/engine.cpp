@@ -110,7 +110,7 @@ extern "C" int prism_create(prism_ctx** out, int32_t device, const char* code_ob
         {&c->f_codec[2], "prism_codec_enc2"}, {&c->f_codec[3], "prism_codec_enc3"},
         {&c->f_codec[4], "prism_codec_dec3"}, {&c->f_codec[5], "prism_codec_dec2"},
         {&c->f_codec[6], "prism_codec_dec1_out"}, {&c->f_codec21, "prism_codec_dec21_out"},
-        {&c->f_enc01, "prism_codec_enc01"},   {&c->f_enc23, "prism_codec_enc23"},
+        {&c->f_enc01, "prism_codec_enc01"},
         {&c->f_attn_ffn[0][0], "prism_attn_d128_ffn"}, {&c->f_attn_ffn[0][1], "prism_attn_d128_w8_ffn"},
         {&c->f_attn_ffn[1][0], "prism_attn_d256_ffn"}, {&c->f_attn_ffn[1][1], "prism_attn_d256_w8_ffn"},
     };

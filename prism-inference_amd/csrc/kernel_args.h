@@ -111,9 +111,9 @@ typedef struct ProjArgs {
     int64_t n_tokens;
 } ProjArgs;
 
-/* Encoder / decoder stages (codec.hpp). Grid: x = ceil(out pixels /
- * (64 * CODEC_TT_<stage>)) (enc0: blocks of CODEC_ENC0_ROWS x CODEC_ENC0_COLS), y = frames;
- * 256 threads. */
+/* Encoder / decoder stages (codec.hpp). Grid of enc1, dec2 and dec1_out: x =
+ * ceil(out pixels / (64 * CODEC_TT_<stage>)) (enc0: blocks of CODEC_ENC0_ROWS x
+ * CODEC_ENC0_COLS), y = frames; 256 threads. The others are persistent. */
 typedef struct CodecArgs {
     const uint16_t* in;   /* the CHW frame (enc0), an NHWC map, or the decoder's coarse map */
     const uint16_t* skip; /* decoder skip map (NHWC), NULL for the encoder */
@@ -128,44 +128,22 @@ typedef struct CodecArgs {
     int32_t out_w, out_h; /* output map (dec1_out: before the PixelShuffle)   */
 } CodecArgs;
 
-/* 16-pixel tiles per wave of each codec stage, and (RS) how many waves share a
- * pixel group, splitting its output channels: a workgroup covers
- * 16 * TT * 4 / RS pixels */
+/* 16-pixel tiles per wave: a workgroup covers 64 * TT pixels */
 #define CODEC_TT_ENC1 4
+#define CODEC_TT_DEC2 4
+#define CODEC_TT_DEC1 2
 /* enc0 output block per workgroup (rows x columns) */
 #define CODEC_ENC0_ROWS 4
 #define CODEC_ENC0_COLS 64
-#define CODEC_TT_ENC2 2
-#define CODEC_TT_ENC3 2
-#define CODEC_TT_DEC3 2
-#define CODEC_TT_DEC2 4
-#define CODEC_TT_DEC1 2
-#define CODEC_RS_ENC1 1
-#define CODEC_RS_ENC2 1
-#define CODEC_RS_ENC3 1
-#define CODEC_RS_DEC3 1
-#define CODEC_RS_DEC2 1
-/* KSP: how many waves of a pixel group split the stage's reduction (its
- * k-steps) instead of its channels; a workgroup then covers
- * 16 * TT * 4 / KSP pixels (RS is 1 for such a stage) */
-#define CODEC_KSP_ENC1 1
-#define CODEC_KSP_ENC2 1
-#define CODEC_KSP_ENC3 4
-#define CODEC_KSP_DEC3 1
-#define CODEC_KSP_DEC2 1
-/* the fused enc0 + enc1 launch: enc1 output block per workgroup (r1 rows x
- * columns; its e0 region is (2 rows + 1) x (2 columns + 1)) */
+/* the persistent launches' blocks, rows x columns: enc0 + enc1 (of r1), enc2
+ * and enc3 (of their output map), dec3 and dec2 + dec1 + output (of r2, r1) */
 #define CODEC_ENC01_ROWS 4
 #define CODEC_ENC01_COLS 32
-/* the fused enc2 + enc3 launch: enc3 output block per workgroup (r3 rows x
- * columns, 32 pixels), and whether the blocks go to the XCDs in bands */
-#define CODEC_ENC23_ROWS 4
-#define CODEC_ENC23_COLS 8
-#define CODEC_ENC23_BAND 1
-/* enc2 over an LDS window (codec_conv_window): output block rows x columns,
- * weight fragments this many k-steps ahead */
-#define CODEC_WIN_ROWS_ENC2 2
-#define CODEC_WIN_COLS_ENC2 16
-#define CODEC_WIN_DW_ENC2 3
+#define CODEC_ENC2_ROWS 4
+#define CODEC_ENC2_COLS 16
+#define CODEC_ENC3_ROWS 4
+#define CODEC_ENC3_COLS 8
+#define CODEC_DEC_ROWS 2
+#define CODEC_DEC_COLS 32
 
 #endif

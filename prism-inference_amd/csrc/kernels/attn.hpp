@@ -325,11 +325,7 @@ __device__ __forceinline__ void attn_window_body(const AttnArgs& a, AttnLds<DIM,
             const bool ok = wy * 8 + (sl >> 3) < a.H && wxx * 8 + (sl & 7) < a.W;
 #pragma unroll
             for (int r = 0; r < UPR; ++r) {
-                f4 v = uacc[r][t];
-                /* max(r16(v), 0) == r16(max(v, 0)): fp16 rounding is monotonic */
-#pragma unroll
-                for (int i = 0; i < 4; ++i) v[i] = fmaxf(v[i], 0.f);
-                const h4 x4 = cvt_h4(v);
+                const h4 x4 = relu_h4(uacc[r][t]);
                 *reinterpret_cast<h4*>(os + sl * LDS + (wave * UPR + r) * 16 + 4 * g) = ok ? x4 : h4{};
             }
         }

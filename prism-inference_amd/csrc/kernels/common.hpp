@@ -197,6 +197,9 @@ __device__ __forceinline__ h4 cvt_h4(f4 v) {
     return h4{(f16)v[0], (f16)v[1], (f16)v[2], (f16)v[3]};
 }
 
+/* max(r16(v), 0), which is r16(max(v, 0)): the rounding is monotonic. */
+__device__ __forceinline__ h4 relu_h4(f4 v) { return __builtin_elementwise_max(cvt_h4(v), h4{}); }
+
 /*
  * LayerNorm of rows into an LDS tile, LPS = DIM/16 lanes per row and 16
  * channels per lane, in two steps so a kernel can put every row load in

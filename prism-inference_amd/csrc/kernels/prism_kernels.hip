@@ -9,6 +9,7 @@
  *   prism_expert_d{256,128}_bm64[_w8], _d256_bm{128,96}  grouped expert FFN
  *   prism_project_{up,down}_d{256,128}             projection adapters (128 <-> dim)
  *   prism_codec_enc{0..3}, prism_codec_dec{3,2}    conv encoder / fused decoder stages
+ *   prism_codec_enc01, prism_codec_dec21_out       the stages fused in the frame
  *   prism_codec_dec1_out                           dec1 + output conv + PixelShuffle + sigmoid
  *   prism_zero_i32                                 clears routing counters
  *   prism_take_counts                              strided counters -> contiguous (stage calls)
@@ -18,6 +19,8 @@
 #include "expert.hpp"
 #include "project.hpp"
 #include "codec.hpp"
+#include "codec_enc.hpp"
+#include "codec_dec.hpp"
 
 /* Routing counters must start at zero; a kernel (not a memset node) keeps
  * the launch safe under stream capture. */

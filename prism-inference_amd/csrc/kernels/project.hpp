@@ -95,13 +95,8 @@ __device__ __forceinline__ void project_body(const ProjArgs& a) {
         for (int t = 0; t < TT; ++t)
 #pragma unroll
             for (int r = 0; r < RT; ++r) {
-                f4 v = acc[r][t];
-                /* max(r16(v), 0) == r16(max(v, 0)): fp16 rounding is monotonic */
-                if constexpr (RELU) {
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) v[i] = fmaxf(v[i], 0.f);
-                }
-                *reinterpret_cast<h4*>(tout + (16 * t + l16) * LO + (wave * RT + r) * 16 + 4 * g) = cvt_h4(v);
+                *reinterpret_cast<h4*>(tout + (16 * t + l16) * LO + (wave * RT + r) * 16 + 4 * g) =
+                    RELU ? relu_h4(acc[r][t]) : cvt_h4(acc[r][t]);
             }
         __syncthreads(); /* the output tile is complete; every wave is done reading tin */
         /* every LDS read first, then the stores (a read under a store's
