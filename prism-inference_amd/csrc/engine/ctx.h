@@ -19,6 +19,7 @@ struct DevBlock {
     uint16_t* wqkv;
     float* bqkv;
     float* bqkv_pad; /* the blob's QKV bias for padded window slots; NULL if LN1 beta = 0 */
+    float* bqkv_blob; /* the same, whatever beta is */
     uint16_t* wo;
     float* bo;
     uint16_t* wr;
@@ -95,6 +96,7 @@ struct prism_ctx {
     int device = 0;
     hipModule_t module = nullptr;
     hipFunction_t f_attn[2][2][5] = {}; /* [d128, d256][4 waves, 8 waves][routed: padded experts / 16] */
+    hipFunction_t f_dense[2][2] = {};    /* [d256][8 waves]: a whole dense chain in one launch */
     hipFunction_t f_attn_ffn[2][2] = {}; /* dense blocks, FFN fused: [d128, d256][4 waves, 8 waves] */
     hipFunction_t f_router[2][4] = {};  /* [dim][padded experts / 16 - 1] */
     hipFunction_t f_expert[2][2] = {};  /* [dim][4 waves, 8 waves], 64-token tiles */

@@ -113,6 +113,8 @@ extern "C" int prism_create(prism_ctx** out, int32_t device, const char* code_ob
         {&c->f_enc01, "prism_codec_enc01"},
         {&c->f_attn_ffn[0][0], "prism_attn_d128_ffn"}, {&c->f_attn_ffn[0][1], "prism_attn_d128_w8_ffn"},
         {&c->f_attn_ffn[1][0], "prism_attn_d256_ffn"}, {&c->f_attn_ffn[1][1], "prism_attn_d256_w8_ffn"},
+        {&c->f_dense[0][0], "prism_chain_d128"}, {&c->f_dense[0][1], "prism_chain_d128_w8"},
+        {&c->f_dense[1][0], "prism_chain_d256"}, {&c->f_dense[1][1], "prism_chain_d256_w8"},
     };
     std::vector<std::pair<hipFunction_t*, std::string>> all;
     for (auto& f : fns) all.emplace_back(f.f, f.name);
@@ -338,7 +340,8 @@ extern "C" int prism_load_weights(prism_ctx* c, const prism_model_desc* d, const
         /* with LN1 beta = 0 the folded bias is the blob's: padded slots need nothing else */
         bool beta1 = false;
         for (int i = 0; i < D && !beta1; ++i) beta1 = (src[offs[b].ln1_b + i] & 0x7fff) != 0;
-        k.bqkv_pad = beta1 ? reinterpret_cast<float*>(base + p.bqkv_pad) : nullptr;
+        k.bqkv_blob = reinterpret_cast<float*>(base + p.bqkv_pad);
+        k.bqkv_pad = beta1 ? k.bqkv_blob : nullptr;
         k.wo = reinterpret_cast<uint16_t*>(base + p.wo);
         k.bo = reinterpret_cast<float*>(base + p.bo);
         k.wr = N > 1 ? reinterpret_cast<uint16_t*>(base + p.wr) : nullptr;
@@ -485,9 +488,11 @@ struct RouteOut {
 /* par: attention launches of about this size that run at the same time (a
  * dense chain's sub-chains; a routed one's run beside the other's experts).
  * ffn: a dense block's FFN runs in the same launch (the window's rows never
- * leave the CU between the two), and `out` receives the block's output */
+ * leave the CU between the two), and `out` receives the block's output.
+ * blocks > 1: that many dense blocks from k on in one launch */
 int enqueue_attn(prism_ctx* c, const DevBlock& k, const uint16_t* in, uint16_t* out, int H, int W, int batch,
-                 hipStream_t s, const RouteOut* route = nullptr, bool up = false, bool ffn = false, int par = 1) {
+                 hipStream_t s, const RouteOut* route = nullptr, bool up = false, bool ffn = false, int par = 1,
+                 int blocks = 1) {
     const int D = c->desc.dim;
     if (ffn && (route || c->desc.n_experts != 1))
         return fail(c, PRISM_ERR_INVALID, "the fused FFN is for dense blocks");
@@ -541,7 +546,17 @@ int enqueue_attn(prism_ctx* c, const DevBlock& k, const uint16_t* in, uint16_t* 
      * launches' windows count together (two dense launches of 256 at once: 162
      * us a four-block chain on 8 waves, 134 on 4). */
     const int w8 = grid * par < (D == 256 ? CU_COUNT + 1 : 2 * CU_COUNT) ? 1 : 0;
-    const hipFunction_t f = ffn ? c->f_attn_ffn[dim_index(D)][w8] : c->f_attn[dim_index(D)][w8][npt];
+    if (blocks > 1) {
+        const DevBlock* const kb = &k;
+        a.n_blocks = blocks;
+        a.block_stride = (const uint8_t*)kb[1].wqkv - (const uint8_t*)kb[0].wqkv; /* the arena repeats per block */
+        /* without beta the blob's bias is the folded one: one answer for all */
+        for (int b = 0; b < blocks; ++b)
+            if (kb[b].bqkv_pad) a.bqkv_pad = kb[0].bqkv_blob;
+    }
+    const hipFunction_t f = blocks > 1 ? c->f_dense[dim_index(D)][w8]
+                            : ffn      ? c->f_attn_ffn[dim_index(D)][w8]
+                                       : c->f_attn[dim_index(D)][w8][npt];
     if (!f) return fail(c, PRISM_ERR_INVALID, "no fused FFN kernel for d%d at %lld windows", D, (long long)grid);
     return launch(c, f, (unsigned)grid, a, s, w8 ? 512u : 256u);
 }
@@ -918,6 +933,19 @@ static int chain_split(const prism_model_desc& d, int batch) {
     return windows > (d.n_experts > 1 ? CHAIN_SPLIT_ROUTED : CHAIN_SPLIT_DENSE) ? std::min(CHAIN_SPLIT, batch) : 1;
 }
 
+/* A dense chain's windows meet no others in any block, so one launch can take
+ * each through all of them with its rows in LDS: no launch, row load or store
+ * between the blocks. At d256 while the windows fit one round of workgroups
+ * (two 4-wave ones per CU): 12 blocks of 135, 270 and 405 windows 195 -> 151,
+ * 267 -> 229 and 339 -> 300 us; of 540 windows, whose second round is nearly
+ * empty for all 12 blocks, 393 and 430; of 1,080, 699 and 739. At d128, whose
+ * windows are short, always: 4 blocks of 135, 540, 1,080 and 2,160 windows
+ * 38 -> 31, 72 -> 57, 104 -> 98 and 182 -> 172 us. */
+static bool dense_one_launch(const prism_model_desc& d, int batch) {
+    const int64_t windows = (int64_t)((d.spatial_w + 7) / 8) * ((d.spatial_h + 7) / 8) * batch;
+    return d.n_experts == 1 && (d.dim == 128 || windows <= 2 * CU_COUNT);
+}
+
 /* Sub-chain j: frames [f0, f0 + nf) through every block, in -> out (this
  * sub-chain's frames). adapted: in and out hold 128-channel rows; block 0's
  * attention runs the up-projection in its prologue and the last block's
@@ -962,7 +990,19 @@ static int enqueue_subchain(prism_ctx* c, const ChainWs& ws, int S, int j, int f
         if (rc) return rc;
     }
     const uint16_t* src = in;
-    for (int b = 0; b < NB; ++b) {
+    int b0 = 0;
+    if (!moe && !tm && S == 1 && dense_one_launch(c->desc, nf)) { /* every block but the one the down-projection follows */
+        b0 = adapted ? NB - 1 : NB;
+        if (b0 > 1) {
+            uint16_t* dst = b0 == NB ? out : scratch;
+            const int rc = enqueue_attn(c, c->blocks[0], src, dst, H, W, nf, s, nullptr, adapted, true, 1, b0);
+            if (rc) return rc;
+            src = dst;
+        } else {
+            b0 = 0;
+        }
+    }
+    for (int b = b0; b < NB; ++b) {
         const DevBlock& k = c->blocks[b];
         const bool first = adapted && b == 0, last = adapted && b == NB - 1;
         uint16_t* dst = last ? out : ((NB - 1 - b) % 2 == 0) ? mid : scratch;
@@ -999,7 +1039,7 @@ static int enqueue_forward_impl(prism_ctx* c, const ChainWs& ws, const uint16_t*
     const int64_t D = adapted ? c->aoffs.in_dim : c->desc.dim; /* channels of in and out */
     c->fwd_tokens = (int64_t)batch * T;
     c->fwd_assign = ws.assign;
-    const int S = chain_split(c->desc, batch);
+    const int S = dense_one_launch(c->desc, batch) ? 1 : chain_split(c->desc, batch);
     if (S == 1) return enqueue_subchain(c, ws, 1, 0, 0, batch, in, out, s, adapted);
     /* fork: sub-chain j > 0 on sub_stream[j-1], sub-chain 0 on s, then join */
     HIP_TRY(c, hipEventRecord(c->ev_fork, s));

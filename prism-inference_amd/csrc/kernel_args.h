@@ -59,6 +59,10 @@ typedef struct AttnArgs {
     const float* ffn_b1;  /* [dim]                                       */
     const uint16_t* ffn_w2; /* packed [dim/16][dim/32]                   */
     const float* ffn_b2;  /* [dim]                                       */
+    /* a dense chain in one launch: blocks, and the bytes from one block's
+     * parameters (every pointer to weights and biases) to the next one's */
+    int64_t block_stride;
+    int32_t n_blocks;
 } AttnArgs;
 
 /* Router stage: at most this many 16-token tiles per wave (the LDS tables

@@ -114,6 +114,8 @@ struct AttnLds {
  * those slots' keys and values need the unfolded bias (a separate
  * instantiation keeps that code, and its branches, out of every other
  * window's instruction schedule). vmask bit s: slot s holds a token.
+ * CHAIN: the body loops over a.n_blocks dense blocks; the raw rows go to os
+ * first, and every block's LN1 reads them there.
  * HALF: slots 32-63 are all padded (the bottom windows of a grid whose
  * height leaves 4 or fewer rows in the last window row, e.g. 68 rows), so
  * token tiles 2 and 3 are never queries, never stored and never routed: only
@@ -123,9 +125,10 @@ struct AttnLds {
  * O, the out-projection, LN1 (and the fused up-projection) and the routing
  * for tiles 0 and 1 only; every stored value is computed as in the full
  * body. */
-template <int DIM, int HD, int NW, int NPT, bool PAD, bool HALF = false, bool FFN = false>
+template <int DIM, int HD, int NW, int NPT, bool PAD, bool HALF = false, bool FFN = false, bool CHAIN = false>
 __device__ __forceinline__ void attn_window_body(const AttnArgs& a, AttnLds<DIM, NPT>& L,
                                                  unsigned long long vmask) {
+    static_assert(!CHAIN || (FFN && NPT == 0), "whole dense blocks");
     constexpr int TQ = HALF ? 2 : 4; /* token tiles that hold tokens */
     static_assert(DIM / HD == 8, "8 heads");
     static_assert(NW == 4 || NW == 8, "4 or 8 waves");
@@ -157,10 +160,10 @@ __device__ __forceinline__ void attn_window_body(const AttnArgs& a, AttnLds<DIM,
     int* const r_e = r_base + 64;                        /* [64] expert per slot     */
     int* const r_rank = r_e + 64;                        /* [64] rank in its bucket  */
 
-    const int lane = lane_id();
+    int lane = lane_id();
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int l16 = lane & 15;
-    const int g = lane >> 4;
+    int l16 = lane & 15;
+    int g = lane >> 4;
 
     const int wg = blockIdx.x;
     const int frame = wg / a.windows_per_frame;
@@ -170,10 +173,7 @@ __device__ __forceinline__ void attn_window_body(const AttnArgs& a, AttnLds<DIM,
     const uint16_t* in = a.in + (int64_t)frame * a.in_frame_elems;
     uint16_t* out = a.out + (int64_t)frame * a.frame_elems;
 
-    const FragSrc src_qkv(a.wqkv, 3u * DIM * DIM * 2u);
-    const FragSrc src_o(a.wo, 1u * DIM * DIM * 2u);
-    const FragSrc src_r(NPT > 0 ? a.wr : a.wo, NPT > 0 ? 16u * NPT * DIM * 2u : 0u);
-    const int loff = lane * 16;
+    int loff = lane * 16;
     /* waves 0-3 route tiles 0-3 of the window (waves w and w+4 tile w % 4
      * when split). Every wave's ring runs into W_r's first fragments (the
      * refills are unconditional: a refill under a wave-dependent branch makes
@@ -238,61 +238,7 @@ __device__ __forceinline__ void attn_window_body(const AttnArgs& a, AttnLds<DIM,
     }
     sched_fence();
 
-    /* weight ring: the first PF fragments */
-    h8 ring[PF];
-#pragma unroll
-    for (int p = 0; p < PF; ++p) ring[p] = attn_frag<DIM, HD, NW, NPT>(src_qkv, src_o, src_r, wave, p, loff);
-    sched_fence();
-
-    /* block chain: clear the next block's counters (its previous reader, that
-     * block's expert stage of the previous chain, has finished) */
-    if (NPT > 0 && a.zero_next && blockIdx.x == 0 && threadIdx.x < a.n_experts)
-        a.zero_next[threadIdx.x * a.count_stride] = 0;
-    /* every parameter is staged here, before LN1. All of a thread's
-     * parameter loads are issued before its first LDS store (a loop of
-     * load-then-store passes waits one L2 round trip per pass); loads retire
-     * in issue order, so the stores wait for the rows, the ring's first
-     * fragments and these loads together: one memory round trip, which LN1
-     * and the QKV GEMM wait for anyway. The barrier after LN1 publishes them
-     * (each wave starts its LN1 as soon as its own rows are in, without
-     * waiting for the other waves' stores) */
-    {
-        constexpr int NQ = (3 * DIM + NT - 1) / NT, NB = (DIM + NT - 1) / NT;
-        constexpr int NR = NPT > 0 ? (16 * NPT + NT - 1) / NT : 0, NRA = NR > 0 ? NR : 1;
-        const int tid = (int)threadIdx.x;
-        float pq[NQ], pp[NQ], pb[NB], pr[NRA];
-#pragma unroll
-        for (int k = 0; k < NQ; ++k) pq[k] = a.bqkv[min(tid + k * NT, 3 * DIM - 1)];
-        if constexpr (PAD) {
-#pragma unroll
-            for (int k = 0; k < NQ; ++k) pp[k] = a.bqkv_pad[min(tid + k * NT, 3 * DIM - 1)];
-        }
-#pragma unroll
-        for (int k = 0; k < NB; ++k) pb[k] = a.bo[min(tid + k * NT, DIM - 1)];
-#pragma unroll
-        for (int k = 0; k < NR; ++k) pr[k] = a.br[min(tid + k * NT, 16 * NPT - 1)];
-        /* the stores are unconditional: a thread past an array's end writes
-           its last entry with the value it holds (the same value), so no
-           branch invites the compiler to sink a load next to its store */
-#pragma unroll
-        for (int k = 0; k < NQ; ++k) {
-            s_bqkv[min(tid + k * NT, 3 * DIM - 1)] = pq[k];
-            if constexpr (PAD) s_bqkv_pad[min(tid + k * NT, 3 * DIM - 1)] = pp[k];
-        }
-#pragma unroll
-        for (int k = 0; k < NB; ++k) s_bo[min(tid + k * NT, DIM - 1)] = pb[k];
-#pragma unroll
-        for (int k = 0; k < NR; ++k) s_br[min(tid + k * NT, 16 * NPT - 1)] = pr[k];
-    }
-    if (!up) {
-        if (lnw) {
-#pragma unroll
-            for (int it = 0; it < IT; ++it) {
-                const int row = (wave * SPW + it * SPI + lane / LPS) * LDS;
-                ln_store<DIM>(rc[it], valid[it], xs + row, os + row); /* os: the raw rows (residual) */
-            }
-        }
-    } else {
+    auto up_project = [&]() {
         /* x = r16(ReLU(W_up e + b_up)) for the window's slots, the same
          * arithmetic as prism_project_up_d* (bias in the accumulator, k-steps
          * in order), into os as the raw rows; padded slots are zero. The 128-
@@ -330,13 +276,106 @@ __device__ __forceinline__ void attn_window_body(const AttnArgs& a, AttnLds<DIM,
             }
         }
         __syncthreads(); /* x complete in os; the staging in xs is dead */
+    };
+    if constexpr (CHAIN) { /* the raw rows into os; every block's LN1 reads them there */
+        if (up) {
+            up_project();
+        } else {
+            if (lnw) {
+#pragma unroll
+                for (int it = 0; it < IT; ++it) {
+                    f16* const row = os + (wave * SPW + it * SPI + lane / LPS) * LDS + (lane % LPS) * 8;
+                    *reinterpret_cast<h8*>(row) = rc[it].a0;
+                    *reinterpret_cast<h8*>(row + DIM / 2) = rc[it].a1;
+                }
+            }
+            __syncthreads();
+        }
+    }
+
+#pragma unroll 1
+    for (int blk = 0; blk < (CHAIN ? a.n_blocks : 1); ++blk) {
+    if constexpr (CHAIN) { /* lane addresses are formed again per block, not held over the loop */
+        asm volatile("" : "+v"(lane));
+        l16 = lane & 15;
+        g = lane >> 4;
+        loff = lane * 16;
+    }
+    /* CHAIN: this block's copy of a parameter (the blocks lie a constant
+     * stride apart); the rows are in os from the second block on */
+    auto par = [&](auto* p) {
+        return CHAIN ? reinterpret_cast<decltype(p)>(reinterpret_cast<const unsigned char*>(p) + blk * a.block_stride) : p;
+    };
+    const FragSrc src_qkv(par(a.wqkv), 3u * DIM * DIM * 2u);
+    const FragSrc src_o(par(a.wo), 1u * DIM * DIM * 2u);
+    const FragSrc src_r(NPT > 0 ? a.wr : a.wo, NPT > 0 ? 16u * NPT * DIM * 2u : 0u);
+    const float *const bqkv = par(a.bqkv), *const bqkv_pad = par(a.bqkv_pad), *const bo = par(a.bo);
+
+    /* weight ring: the first PF fragments */
+    h8 ring[PF];
+#pragma unroll
+    for (int p = 0; p < PF; ++p) ring[p] = attn_frag<DIM, HD, NW, NPT>(src_qkv, src_o, src_r, wave, p, loff);
+    sched_fence();
+
+    /* block chain: clear the next block's counters (its previous reader, that
+     * block's expert stage of the previous chain, has finished) */
+    if (NPT > 0 && a.zero_next && blockIdx.x == 0 && threadIdx.x < a.n_experts)
+        a.zero_next[threadIdx.x * a.count_stride] = 0;
+    /* every parameter is staged here, before LN1. All of a thread's
+     * parameter loads are issued before its first LDS store (a loop of
+     * load-then-store passes waits one L2 round trip per pass); loads retire
+     * in issue order, so the stores wait for the rows, the ring's first
+     * fragments and these loads together: one memory round trip, which LN1
+     * and the QKV GEMM wait for anyway. The barrier after LN1 publishes them
+     * (each wave starts its LN1 as soon as its own rows are in, without
+     * waiting for the other waves' stores) */
+    {
+        constexpr int NQ = (3 * DIM + NT - 1) / NT, NB = (DIM + NT - 1) / NT;
+        constexpr int NR = NPT > 0 ? (16 * NPT + NT - 1) / NT : 0, NRA = NR > 0 ? NR : 1;
+        const int tid = (int)threadIdx.x;
+        float pq[NQ], pp[NQ], pb[NB], pr[NRA];
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) pq[k] = bqkv[min(tid + k * NT, 3 * DIM - 1)];
+        if constexpr (PAD) {
+#pragma unroll
+            for (int k = 0; k < NQ; ++k) pp[k] = bqkv_pad[min(tid + k * NT, 3 * DIM - 1)];
+        }
+#pragma unroll
+        for (int k = 0; k < NB; ++k) pb[k] = bo[min(tid + k * NT, DIM - 1)];
+#pragma unroll
+        for (int k = 0; k < NR; ++k) pr[k] = a.br[min(tid + k * NT, 16 * NPT - 1)];
+        /* the stores are unconditional: a thread past an array's end writes
+           its last entry with the value it holds (the same value), so no
+           branch invites the compiler to sink a load next to its store */
+#pragma unroll
+        for (int k = 0; k < NQ; ++k) {
+            s_bqkv[min(tid + k * NT, 3 * DIM - 1)] = pq[k];
+            if constexpr (PAD) s_bqkv_pad[min(tid + k * NT, 3 * DIM - 1)] = pp[k];
+        }
+#pragma unroll
+        for (int k = 0; k < NB; ++k) s_bo[min(tid + k * NT, DIM - 1)] = pb[k];
+#pragma unroll
+        for (int k = 0; k < NR; ++k) s_br[min(tid + k * NT, 16 * NPT - 1)] = pr[k];
+    }
+    if (!CHAIN && !up) {
         if (lnw) {
 #pragma unroll
             for (int it = 0; it < IT; ++it) {
                 const int row = (wave * SPW + it * SPI + lane / LPS) * LDS;
+                ln_store<DIM>(rc[it], valid[it], xs + row, os + row); /* os: the raw rows (residual) */
+            }
+        }
+    } else {
+        if constexpr (!CHAIN) up_project();
+        if (lnw) { /* the raw rows are in os */
+#pragma unroll
+            for (int it = 0; it < IT; ++it) {
+                const int row = (wave * SPW + it * SPI + lane / LPS) * LDS;
                 const int ca = (lane % LPS) * 8;
-                const RowChunk xr{*reinterpret_cast<const h8*>(os + row + ca),
-                                  *reinterpret_cast<const h8*>(os + row + ca + DIM / 2)};
+                RowChunk xr{*reinterpret_cast<const h8*>(os + row + ca),
+                            *reinterpret_cast<const h8*>(os + row + ca + DIM / 2)};
+                /* what a padded slot's row became over the blocks may overflow */
+                if (CHAIN && !valid[it]) xr = RowChunk{};
                 ln_store<DIM>(xr, valid[it], xs + row, nullptr);
             }
         }
@@ -684,7 +723,8 @@ __device__ __forceinline__ void attn_window_body(const AttnArgs& a, AttnLds<DIM,
         static_assert(NPT == 0, "dense blocks only");
         constexpr int RT = DIM / 16 / NW; /* hidden / output row tiles per wave */
         static_assert(RT >= 1, "FFN shape");
-        const FragSrc w1(a.ffn_w1, DIM * DIM * 2u), w2(a.ffn_w2, DIM * DIM * 2u);
+        const FragSrc w1(par(a.ffn_w1), DIM * DIM * 2u), w2(par(a.ffn_w2), DIM * DIM * 2u);
+        const float *const fb1 = par(a.ffn_b1), *const fb2 = par(a.ffn_b2);
         /* the wave's weight stream: W1 then W2, k-step-major over its RT row
          * tiles, through a ring of FR fragments (all of W1 when that is at
          * most 16 fragments, W2 then refilling the slots GEMM1 frees; else
@@ -715,7 +755,7 @@ __device__ __forceinline__ void attn_window_body(const AttnArgs& a, AttnLds<DIM,
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
             const int ch = (wave * RT + r) * 16 + 4 * g;
-            const f4 bb = {a.ffn_b1[ch], a.ffn_b1[ch + 1], a.ffn_b1[ch + 2], a.ffn_b1[ch + 3]};
+            const f4 bb = {fb1[ch], fb1[ch + 1], fb1[ch + 2], fb1[ch + 3]};
 #pragma unroll
             for (int t = 0; t < 4; ++t) facc[r][t] = bb;
         }
@@ -746,7 +786,7 @@ __device__ __forceinline__ void attn_window_body(const AttnArgs& a, AttnLds<DIM,
 #pragma unroll
         for (int r = 0; r < RT; ++r) {
             const int ch = (wave * RT + r) * 16 + 4 * g;
-            const f4 bb = {a.ffn_b2[ch], a.ffn_b2[ch + 1], a.ffn_b2[ch + 2], a.ffn_b2[ch + 3]};
+            const f4 bb = {fb2[ch], fb2[ch + 1], fb2[ch + 2], fb2[ch + 3]};
 #pragma unroll
             for (int t = 0; t < TQ; ++t) {
                 const h4 u = cvt_h4(facc[r][t]); /* r16(W1 hn + b1) */
@@ -797,10 +837,12 @@ __device__ __forceinline__ void attn_window_body(const AttnArgs& a, AttnLds<DIM,
         __syncthreads(); /* the block's output tile complete in os */
     }
 
-    if constexpr (NPT == 0 || NW == 8) store_rows();
+    if constexpr (NPT == 0 || NW == 8)
+        if (!CHAIN || blk == a.n_blocks - 1) store_rows();
+    } /* blocks */
 }
 
-template <int DIM, int HD, int NW, int NPT, bool FFN = false>
+template <int DIM, int HD, int NW, int NPT, bool FFN = false, bool CHAIN = false>
 __device__ __forceinline__ void attn_window(const AttnArgs& a, AttnLds<DIM, NPT>& L) {
     const int wi = blockIdx.x % a.windows_per_frame;
     const int wy = wi / a.wx, wxx = wi - (wi / a.wx) * a.wx;
@@ -809,13 +851,13 @@ __device__ __forceinline__ void attn_window(const AttnArgs& a, AttnLds<DIM, NPT>
     const bool half = (vmask >> 32) == 0ull; /* uniform */
     if (a.bqkv_pad != nullptr && vmask != ~0ull) {
         if (half)
-            attn_window_body<DIM, HD, NW, NPT, true, true, FFN>(a, L, vmask);
+            attn_window_body<DIM, HD, NW, NPT, true, true, FFN, CHAIN>(a, L, vmask);
         else
-            attn_window_body<DIM, HD, NW, NPT, true, false, FFN>(a, L, vmask);
+            attn_window_body<DIM, HD, NW, NPT, true, false, FFN, CHAIN>(a, L, vmask);
     } else if (half) {
-        attn_window_body<DIM, HD, NW, NPT, false, true, FFN>(a, L, vmask);
+        attn_window_body<DIM, HD, NW, NPT, false, true, FFN, CHAIN>(a, L, vmask);
     } else {
-        attn_window_body<DIM, HD, NW, NPT, false, false, FFN>(a, L, vmask);
+        attn_window_body<DIM, HD, NW, NPT, false, false, FFN, CHAIN>(a, L, vmask);
     }
 }
 
@@ -859,5 +901,24 @@ extern "C" __global__ void __launch_bounds__(256, 2) prism_attn_d256_ffn(AttnArg
 extern "C" __global__ void __launch_bounds__(512, 1) prism_attn_d256_w8_ffn(AttnArgs a) {
     __shared__ AttnLds<256, 0> lds;
     attn_window<256, 32, 8, 0, true>(a, lds);
+}
+/* a whole dense chain in one launch: windows are never shifted, so a window's
+ * 64 tokens meet no others in any block, and its rows stay in LDS from the
+ * first block's input to the last one's output */
+extern "C" __global__ void __launch_bounds__(512, 4) prism_chain_d128_w8(AttnArgs a) {
+    __shared__ AttnLds<128, 0> lds;
+    attn_window<128, 16, 8, 0, true, true>(a, lds);
+}
+extern "C" __global__ void __launch_bounds__(512, 2) prism_chain_d256_w8(AttnArgs a) {
+    __shared__ AttnLds<256, 0> lds;
+    attn_window<256, 32, 8, 0, true, true>(a, lds);
+}
+extern "C" __global__ void __launch_bounds__(256, 2) prism_chain_d256(AttnArgs a) {
+    __shared__ AttnLds<256, 0> lds;
+    attn_window<256, 32, 4, 0, true, true>(a, lds);
+}
+extern "C" __global__ void __launch_bounds__(256, 3) prism_chain_d128(AttnArgs a) {
+    __shared__ AttnLds<128, 0> lds;
+    attn_window<128, 16, 4, 0, true, true>(a, lds);
 }
 #undef PRISM_ATTN_KERNELS

@@ -1,6 +1,7 @@
 """The chain's choice of kernels and sub-chains by the number of windows: 8-wave
 workgroups up to one per CU (256 windows at d256, 511 at d128),
-4-wave ones above; two sub-chains above 192 windows (MoE) or 512 (dense). Frames never interact, so a frame's
+4-wave ones above; two sub-chains above 192 windows (MoE) or 512 (dense); a
+dense chain in one launch (d128, and up to 512 windows at d256). Frames never interact, so a frame's
 output is the same bits whichever side of an edge its batch lies on."""
 import numpy as np
 import pytest
@@ -40,3 +41,35 @@ def test_frame_is_the_same_in_every_batch(hip, engine, device_arena, name, batch
                 engine.forward(dx.ptr + (b - 1) * n * d * 2, dy.ptr, 1, graph=graph)
                 hip.sync()
                 assert (hip.download(np.empty(n * d, np.uint16), dy.ptr) == y[b - 1]).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,batch", [("std256", 1), ("std256", 5), ("dense128", 1), ("dense128", 8)])
+@pytest.mark.parametrize("beta_blocks", [(), (0,), (2,), (0, 1, 2)])
+def test_dense_chain_in_one_launch(hip, engine, device_arena, name, batch, beta_blocks):
+    """Blocks with and without an LN1 beta (whose padded window slots need the
+    blob's own bias) in one launch: the stage calls' output bit for bit."""
+    H, W, nb = 61, 59, 3
+    cfg = P.CONFIGS[name]
+    desc = cfg.desc(n_blocks=nb, H=H, W=W)
+    blob, offs = P.synth_weights(desc, seed=7, routing=cfg.routing)
+    d, n = cfg.dim, batch * H * W
+    for b in beta_blocks:
+        beta = np.random.default_rng(b).normal(0, 0.2, d).astype(np.float16)
+        blob[offs[b].ln1_b:offs[b].ln1_b + d] = beta.view(np.uint16)
+    engine.load_weights(desc, blob, offs)
+    x = P.synth_features(cfg, batch=batch, H=H, W=W, seed=8).reshape(-1)
+    dx, dy, feats = device_arena(x.nbytes), device_arena(x.nbytes), device_arena(3 * x.nbytes)
+    hip.upload(dx.ptr, x)
+    hip.upload(feats.ptr, x)
+    print(f"[dispatch] {name} batch {batch} beta in blocks {beta_blocks}", flush=True)
+    engine.forward(dx.ptr, dy.ptr, batch)
+    cur, nxt = 0, 2 * n * d
+    for b in range(nb):
+        assert engine.attn(engine.attn_push(b, cur, n * d), feats.ptr, batch) == 0, engine.error()
+        assert engine.experts(engine.expert_push(b, H * W, n * d, nxt), feats.ptr, None, batch) == 0, engine.error()
+        cur, nxt = nxt, cur
+    hip.sync()
+    got = hip.download(np.empty(n * d, np.uint16), dy.ptr)
+    ref = hip.download(np.empty(n * d, np.uint16), feats.ptr + cur * 2)
+    assert (got == ref).all(), f"{int((got != ref).sum())} values differ"
