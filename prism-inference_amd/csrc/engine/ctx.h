@@ -67,10 +67,11 @@ static constexpr int EXPERT_WIDE_MIN_TILES = 512;
  * sets wnt_blocks). */
 static constexpr int64_t WEIGHT_CACHE_KEEP = 224ll << 20;
 /* Workgroups of a projection stage launch (persistent, 64-token tiles in a
- * loop; the d256 kernels' 210-220 VGPRs allow two per CU). At batch 16,
- * 68x120, up 128->256: 512 workgroups 18.5 us, 384 20.6, 256 23.5, 1024
- * 21.8 (one workgroup per tile: 20.5). */
+ * loop, two per CU); at d256 up to PROJ_SINGLE_MAX tiles go one to a
+ * workgroup. Both d256 launches, 765 tiles: 19.1 us on 512 workgroups, 18.3 on
+ * 765; 2,040 tiles: 41.5 on 512, 43.7 on 768. */
 static constexpr int PROJ_GRID_MAX = 512;
+static constexpr int PROJ_SINGLE_MAX = 768;
 
 /* Attention keys all 64 slots of a window. The reference keys the first
  * min(64, n_tokens) slots in slot order (split2_qkv_attn_d256.comp.glsl:33,60),

@@ -644,9 +644,11 @@ int enqueue_project(prism_ctx* c, bool up, const uint16_t* in, uint16_t* out, in
     a.n_tokens = n;
     const int64_t tiles = (n + 63) / 64;
     if (tiles <= 0 || tiles > 0x7fffffff) return fail(c, PRISM_ERR_INVALID, "projection tiles %lld out of range", (long long)tiles);
-    /* persistent workgroups, each looping over 64-token tiles */
-    const int64_t grid = std::min<int64_t>(tiles, PROJ_GRID_MAX);
-    return launch(c, c->f_proj[dim_index(c->desc.dim)][up ? 0 : 1], (unsigned)grid, a, s);
+    /* persistent workgroups looping over 64-token tiles; at d256 a tile each
+     * while they are few (ctx.h) */
+    const bool d256 = c->desc.dim == 256;
+    const int64_t grid = d256 && tiles <= PROJ_SINGLE_MAX ? tiles : std::min<int64_t>(tiles, PROJ_GRID_MAX);
+    return launch(c, c->f_proj[dim_index(c->desc.dim)][up ? 0 : 1], (unsigned)grid, a, s, d256 ? 512u : 256u);
 }
 
 /* which: 0 = attention (qkv_w), 1 = router (router_w), 2 = experts (exp_w1) */

@@ -7,25 +7,28 @@
  * tiles: C^T = W * X^T with the packed weights as the A operand. A tile's 64
  * token rows are one contiguous block in and one out (HWC): they pass through
  * an LDS tile as whole rows, 16 bytes per lane, and the B fragments (token
- * 16t + l16, channels 32ks + 8g .. +7) are read from there. Workgroup = 4
- * waves; wave w computes output rows [w*OUT/4, +OUT/4) of a tile's 64
+ * 16t + l16, channels 32ks + 8g .. +7) are read from there. Workgroup =
+ * NW waves; wave w computes output rows [w*OUT/NW, +OUT/NW) of a tile's 64
  * tokens, accumulators starting at the bias. Persistent: workgroup b takes
  * tiles b, b + G, b + 2G, ... (G = the grid), holds its waves' weight
  * fragments in registers across them, and requests the next tile's rows
- * before the current tile's MFMAs.
+ * before the current tile's MFMAs. d256 on 8 waves (112 VGPRs, 16 waves per
+ * CU instead of 8: both launches of 4 and 6 frames of 68x120 15.2 -> 13.9 and
+ * 19.9 -> 18.3 us), d128 on 4 (8 measured 4 % slower).
  */
 #pragma once
 #include "common.hpp"
 
-template <int IN, int OUT, bool RELU>
+template <int IN, int OUT, bool RELU, int NW>
 __device__ __forceinline__ void project_body(const ProjArgs& a) {
     constexpr int KS = IN / 32;  /* k-steps                     */
-    constexpr int RT = OUT / 64; /* 16-row output tiles per wave */
+    constexpr int NT = 64 * NW;  /* threads                     */
+    constexpr int RT = OUT / 16 / NW; /* 16-row output tiles per wave */
     constexpr int TT = 4;        /* 16-token tiles per token tile */
     constexpr int LI = IN + 8, LO = OUT + 8;  /* padded LDS rows (halfs) */
-    constexpr int EI = 64 * IN / 8 / 256;     /* 16-byte input chunks per thread  */
-    constexpr int EO = 64 * OUT / 8 / 256;    /* 16-byte output chunks per thread */
-    static_assert(IN % 32 == 0 && OUT % 64 == 0 && EI >= 1 && EO >= 1, "shape");
+    constexpr int EI = 64 * IN / 8 / NT;      /* 16-byte input chunks per thread  */
+    constexpr int EO = 64 * OUT / 8 / NT;     /* 16-byte output chunks per thread */
+    static_assert(IN % 32 == 0 && RT >= 1 && EI >= 1 && EO >= 1, "shape");
     __shared__ __attribute__((aligned(16))) f16 tin[64 * LI];
     __shared__ __attribute__((aligned(16))) f16 tout[64 * LO];
 
@@ -44,7 +47,7 @@ __device__ __forceinline__ void project_body(const ProjArgs& a) {
         const int rows = (int)min<int64_t>(64, a.n_tokens - tok0);
 #pragma unroll
         for (int k = 0; k < EI; ++k) {
-            const int q = threadIdx.x + 256 * k, r = q / (IN / 8), c8 = (q % (IN / 8)) * 8;
+            const int q = threadIdx.x + NT * k, r = q / (IN / 8), c8 = (q % (IN / 8)) * 8;
             const h8 v = *reinterpret_cast<const h8*>(a.in + (tok0 + min(r, rows - 1)) * IN + c8);
             x[k] = r < rows ? v : h8{};
         }
@@ -71,7 +74,7 @@ __device__ __forceinline__ void project_body(const ProjArgs& a) {
         const int rows = (int)min<int64_t>(64, a.n_tokens - tok0);
 #pragma unroll
         for (int k = 0; k < EI; ++k) {
-            const int q = threadIdx.x + 256 * k, r = q / (IN / 8), c8 = (q % (IN / 8)) * 8;
+            const int q = threadIdx.x + NT * k, r = q / (IN / 8), c8 = (q % (IN / 8)) * 8;
             *reinterpret_cast<h8*>(tin + r * LI + c8) = xin[k];
         }
         __syncthreads(); /* the input tile is in; the previous tile's output rows are out of tout */
@@ -104,27 +107,27 @@ __device__ __forceinline__ void project_body(const ProjArgs& a) {
         h8 yo[EO];
 #pragma unroll
         for (int k = 0; k < EO; ++k) {
-            const int q = threadIdx.x + 256 * k, r = q / (OUT / 8), c8 = (q % (OUT / 8)) * 8;
+            const int q = threadIdx.x + NT * k, r = q / (OUT / 8), c8 = (q % (OUT / 8)) * 8;
             yo[k] = *reinterpret_cast<const h8*>(tout + r * LO + c8);
         }
 #pragma unroll
         for (int k = 0; k < EO; ++k) {
-            const int q = threadIdx.x + 256 * k, r = q / (OUT / 8), c8 = (q % (OUT / 8)) * 8;
+            const int q = threadIdx.x + NT * k, r = q / (OUT / 8), c8 = (q % (OUT / 8)) * 8;
             if (r < rows) *reinterpret_cast<h8*>(a.out + (tok0 + r) * OUT + c8) = yo[k];
         }
     }
 }
 
 /* up: encoder channels (128) -> model dim, ReLU; down: model dim -> 128 */
-extern "C" __global__ void __launch_bounds__(256, 2) prism_project_up_d256(ProjArgs a) {
-    project_body<128, 256, true>(a);
+extern "C" __global__ void __launch_bounds__(512, 4) prism_project_up_d256(ProjArgs a) {
+    project_body<128, 256, true, 8>(a);
 }
-extern "C" __global__ void __launch_bounds__(256, 2) prism_project_down_d256(ProjArgs a) {
-    project_body<256, 128, false>(a);
+extern "C" __global__ void __launch_bounds__(512, 4) prism_project_down_d256(ProjArgs a) {
+    project_body<256, 128, false, 8>(a);
 }
 extern "C" __global__ void __launch_bounds__(256, 2) prism_project_up_d128(ProjArgs a) {
-    project_body<128, 128, true>(a);
+    project_body<128, 128, true, 4>(a);
 }
 extern "C" __global__ void __launch_bounds__(256, 2) prism_project_down_d128(ProjArgs a) {
-    project_body<128, 128, false>(a);
+    project_body<128, 128, false, 4>(a);
 }
