@@ -104,7 +104,6 @@ struct prism_ctx {
     hipFunction_t f_expert_wide = nullptr; /* d256, 128-token tiles */
     hipFunction_t f_expert_wide96 = nullptr; /* d256, 96-token tiles (large stage calls) */
     hipFunction_t f_zero = nullptr;
-    hipFunction_t f_take = nullptr;
     hipFunction_t f_proj[2][2] = {};    /* [dim][up, down] */
     hipFunction_t f_codec[7] = {};     /* enc0..enc3, dec3, dec2, dec1_out */
     hipFunction_t f_codec21 = nullptr; /* dec2 + dec1_out in one launch (the decoder's last two stages) */

@@ -103,7 +103,7 @@ extern "C" int prism_create(prism_ctx** out, int32_t device, const char* code_ob
         {&c->f_expert[0][0], "prism_expert_d128_bm64"},  {&c->f_expert[1][0], "prism_expert_d256_bm64"},
         {&c->f_expert[0][1], "prism_expert_d128_bm64_w8"}, {&c->f_expert[1][1], "prism_expert_d256_bm64_w8"},
         {&c->f_expert_wide, "prism_expert_d256_bm128"}, {&c->f_expert_wide96, "prism_expert_d256_bm96"},
-        {&c->f_zero, "prism_zero_i32"}, {&c->f_take, "prism_take_counts"},
+        {&c->f_zero, "prism_zero_i32"},
         {&c->f_proj[0][0], "prism_project_up_d128"},   {&c->f_proj[0][1], "prism_project_down_d128"},
         {&c->f_proj[1][0], "prism_project_up_d256"},   {&c->f_proj[1][1], "prism_project_down_d256"},
         {&c->f_codec[0], "prism_codec_enc0"}, {&c->f_codec[1], "prism_codec_enc1"},
@@ -483,6 +483,7 @@ struct RouteOut {
     int32_t* perm;
     int32_t count_stride;
     int32_t* zero_next; /* counters this launch clears for a later one, or NULL */
+    RouteTake take;     /* stage calls: where the totals go */
 };
 
 /* par: attention launches of about this size that run at the same time (a
@@ -533,6 +534,7 @@ int enqueue_attn(prism_ctx* c, const DevBlock& k, const uint16_t* in, uint16_t* 
         a.cap = (int32_t)((int64_t)batch * H * W);
         a.count_stride = route->count_stride;
         a.zero_next = route->zero_next;
+        a.take = route->take;
     }
     const int64_t grid = (int64_t)a.windows_per_frame * batch;
     if (grid <= 0 || grid > 0x7fffffff) return fail(c, PRISM_ERR_INVALID, "attention grid %lld out of range", (long long)grid);
@@ -570,7 +572,7 @@ int enqueue_zero(prism_ctx* c, int32_t* p, int32_t n, hipStream_t s) {
 }
 
 int enqueue_router(prism_ctx* c, const DevBlock& k, const uint16_t* in, int32_t* assign, int32_t* counts,
-                   int32_t* perm, int64_t n, hipStream_t s, int32_t count_stride) {
+                   int32_t* perm, int64_t n, hipStream_t s, int32_t count_stride, const RouteTake& take) {
     const int N = c->desc.n_experts;
     RouterArgs a{};
     a.in = in;
@@ -584,6 +586,7 @@ int enqueue_router(prism_ctx* c, const DevBlock& k, const uint16_t* in, int32_t*
     a.np = round16(N);
     a.cap = (int32_t)n;
     a.count_stride = count_stride;
+    a.take = take;
     /* tiles per wave for about 512 workgroups (two per CU): one tile per wave
      * at frame scale, 4 at batch 16 (measured 8.9 / 22.2 us; more, smaller
      * workgroups each copy W_r into LDS, fewer leave CUs idle) */
@@ -728,30 +731,21 @@ extern "C" int prism_attn(prism_ctx* c, const prism_attn_push* p, void* features
 
 /* The routing stage calls count into a private row, counters 256 B apart as
  * in the chain (every workgroup adds to them; adjacent counters would
- * serialise those atomics), and prism_take_counts then moves the totals to
- * the caller's contiguous counts, clearing the row for the next call. */
+ * serialise those atomics); the launch's last workgroup moves the totals to
+ * the caller's contiguous counts and leaves the row and its tickets (behind the
+ * row) at zero for the next call. */
+static constexpr int STAGE_ROW = 64 * CHAIN_COUNT_STRIDE, STAGE_ELEMS = STAGE_ROW + 9 * ROUTE_TICKET_STRIDE;
 static int stage_counts_begin(prism_ctx* c, hipStream_t s) {
     if (!c->stage_counts) {
-        const size_t bytes = sizeof(int32_t) * 64 * CHAIN_COUNT_STRIDE;
+        const size_t bytes = sizeof(int32_t) * STAGE_ELEMS;
         HIP_TRY(c, hipMalloc((void**)&c->stage_counts, bytes));
         HIP_TRY(c, hipMemset(c->stage_counts, 0, bytes));
     }
     if (c->stage_dirty) {
-        const int rc = enqueue_zero(c, c->stage_counts, 64 * CHAIN_COUNT_STRIDE, s);
+        const int rc = enqueue_zero(c, c->stage_counts, STAGE_ELEMS, s);
         if (rc) return rc;
-        c->stage_dirty = false;
     }
-    c->stage_dirty = true; /* until stage_counts_take has been enqueued */
-    return PRISM_OK;
-}
-
-static int stage_counts_take(prism_ctx* c, int32_t* dst, int32_t n, hipStream_t s) {
-    int32_t* src = c->stage_counts;
-    int32_t stride = CHAIN_COUNT_STRIDE;
-    void* params[] = {&src, &stride, &dst, &n};
-    const hipError_t e = hipModuleLaunchKernel(c->f_take, 1, 1, 1, 64, 1, 1, 0, s, params, nullptr);
-    if (e != hipSuccess) return fail(c, PRISM_ERR_HIP, "hipModuleLaunchKernel(take counts): %s", hipGetErrorString(e));
-    c->stage_dirty = false;
+    c->stage_dirty = true; /* until the launch that leaves the row clean has been enqueued */
     return PRISM_OK;
 }
 
@@ -766,9 +760,10 @@ extern "C" int prism_router(prism_ctx* c, const prism_router_push* p, const void
     if (rc) return rc;
     const uint16_t* f = static_cast<const uint16_t*>(features);
     rc = enqueue_router(c, *k, f + p->input_offset, aux + p->assignment_offset, c->stage_counts,
-                        aux + p->perm_offset, (int64_t)batch * p->n_tokens, s, CHAIN_COUNT_STRIDE);
-    if (rc) return rc;
-    return stage_counts_take(c, aux + p->count_offset, p->n_experts, s);
+                        aux + p->perm_offset, (int64_t)batch * p->n_tokens, s, CHAIN_COUNT_STRIDE,
+                        RouteTake{c->stage_counts + STAGE_ROW, aux + p->count_offset});
+    c->stage_dirty = rc != PRISM_OK;
+    return rc;
 }
 
 extern "C" int prism_attn_route(prism_ctx* c, const prism_attn_push* pa, const prism_router_push* pr, void* features,
@@ -787,10 +782,11 @@ extern "C" int prism_attn_route(prism_ctx* c, const prism_attn_push* pa, const p
     rc = stage_counts_begin(c, s);
     if (rc) return rc;
     uint16_t* f = static_cast<uint16_t*>(features);
-    const RouteOut ro{aux + pr->assignment_offset, c->stage_counts, aux + pr->perm_offset, CHAIN_COUNT_STRIDE, nullptr};
+    const RouteOut ro{aux + pr->assignment_offset, c->stage_counts, aux + pr->perm_offset, CHAIN_COUNT_STRIDE, nullptr,
+                      RouteTake{c->stage_counts + STAGE_ROW, aux + pr->count_offset}};
     rc = enqueue_attn(c, *ka, f + pa->input_offset, f + pa->output_offset, pa->spatial_h, pa->spatial_w, batch, s, &ro);
-    if (rc) return rc;
-    return stage_counts_take(c, aux + pr->count_offset, pr->n_experts, s);
+    c->stage_dirty = rc != PRISM_OK;
+    return rc;
 }
 
 extern "C" int prism_experts(prism_ctx* c, const prism_expert_push* p, void* features, int32_t* aux, int32_t batch,
@@ -1011,7 +1007,7 @@ static int enqueue_subchain(prism_ctx* c, const ChainWs& ws, int S, int j, int f
         if (moe) {
             int32_t* counts = counts0 + (size_t)b * row;
             const RouteOut ro{ws.assign + (size_t)b * n_all + t0, counts, perm, CHAIN_COUNT_STRIDE,
-                              NB > 1 ? counts0 + (size_t)((b + 1) % NB) * row : nullptr};
+                              NB > 1 ? counts0 + (size_t)((b + 1) % NB) * row : nullptr, RouteTake{}};
             int rc = enqueue_attn(c, k, src, attn, H, W, nf, s, &ro, first);
             if (!rc) rc = timer_mark(c, tm, 0, s);
             if (!rc)

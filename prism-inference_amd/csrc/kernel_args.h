@@ -21,6 +21,14 @@
 #define PRISM_KERNEL_ARGS_H
 #include <stdint.h>
 
+/* Where a routing stage call's totals go (route.hpp); NULL in the chain, whose
+ * expert launches read the counters in place. */
+#define ROUTE_TICKET_STRIDE 64
+typedef struct RouteTake {
+    int32_t* ticket; /* 9 ints ROUTE_TICKET_STRIDE apart, zero on entry and exit; NULL = leave the counters */
+    int32_t* counts; /* [n_experts] contiguous */
+} RouteTake;
+
 typedef struct AttnArgs {
     const uint16_t* in;   /* features + input_offset (fp16 HWC)         */
     uint16_t* out;        /* features + output_offset                   */
@@ -63,6 +71,7 @@ typedef struct AttnArgs {
      * parameters (every pointer to weights and biases) to the next one's */
     int64_t block_stride;
     int32_t n_blocks;
+    RouteTake take; /* routed kernels */
 } AttnArgs;
 
 /* Router stage: at most this many 16-token tiles per wave (the LDS tables
@@ -82,6 +91,7 @@ typedef struct RouterArgs {
     int32_t cap;          /* bucket capacity = n_tokens                    */
     int32_t tiles_per_wave; /* 16-token tiles per wave: WG = 64*tiles tokens */
     int32_t count_stride; /* ints between counters                         */
+    RouteTake take;
 } RouterArgs;
 
 typedef struct ExpertArgs {

@@ -640,6 +640,7 @@ __device__ __forceinline__ void attn_window_body(const AttnArgs& a, AttnLds<DIM,
         }
     };
 
+    int ticket = 0;
     /* ---- 5. fused routing (moe_router.comp.glsl:24-52 + counting sort) -- */
     if constexpr (NPT > 0) {
         auto rfrag = [&](int rt, int ks) {
@@ -700,6 +701,7 @@ __device__ __forceinline__ void attn_window_body(const AttnArgs& a, AttnLds<DIM,
             r_base[threadIdx.x] = c ? atomicAdd(&a.counts[threadIdx.x * a.count_stride], c) : 0;
         }
         __syncthreads();
+        ticket = route_ticket(a.take);
         if (threadIdx.x < 64) {
             const int ty = wy * 8 + (threadIdx.x >> 3), tx = wxx * 8 + (threadIdx.x & 7);
             if (ty < a.H && tx < a.W) {
@@ -839,6 +841,7 @@ __device__ __forceinline__ void attn_window_body(const AttnArgs& a, AttnLds<DIM,
 
     if constexpr (NPT == 0 || NW == 8)
         if (!CHAIN || blk == a.n_blocks - 1) store_rows();
+    if constexpr (NPT > 0) route_take(a.take, ticket, a.counts, a.count_stride, a.n_experts, r_hist);
     } /* blocks */
 }
 

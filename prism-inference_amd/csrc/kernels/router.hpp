@@ -103,6 +103,7 @@ __device__ __forceinline__ void router_body(const RouterArgs& a) {
         base[threadIdx.x] = c ? atomicAdd(&a.counts[threadIdx.x * a.count_stride], c) : 0;
     }
     __syncthreads();
+    const int ticket = route_ticket(a.take);
     for (int j = threadIdx.x; j < wg_tokens; j += 256) {
         const int token = tok_wg0 + j;
         if (token < a.n_tokens) {
@@ -112,6 +113,7 @@ __device__ __forceinline__ void router_body(const RouterArgs& a) {
             if (slot < a.cap) a.perm[(int64_t)e * a.cap + slot] = token;
         }
     }
+    route_take(a.take, ticket, a.counts, a.count_stride, a.n_experts, hist); /* hist is dead since the base atomics */
 }
 
 #define PRISM_ROUTER_KERNEL(D, NPT)                                                                 \

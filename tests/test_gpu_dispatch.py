@@ -73,3 +73,37 @@ def test_dense_chain_in_one_launch(hip, engine, device_arena, name, batch, beta_
     got = hip.download(np.empty(n * d, np.uint16), dy.ptr)
     ref = hip.download(np.empty(n * d, np.uint16), feats.ptr + cur * 2)
     assert (got == ref).all(), f"{int((got != ref).sum())} values differ"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name", ["moe16", "moe64"])
+@pytest.mark.parametrize("H,W,batch", [
+    (8, 8, 1),      # one workgroup: one ticket group
+    (8, 56, 1),     # 7 and 9 workgroups: fewer groups than 8, one of them with two tickets
+    (8, 72, 1),
+    (17, 61, 3),    # 72 windows: 8 groups of 9
+    (61, 59, 5),    # 320: 4-wave attention
+])
+def test_stage_counts_by_the_last_workgroup(hip, engine, device_arena, name, H, W, batch):
+    """The routing stage calls' totals, moved by the launch's last workgroup:
+    exact on every call, each of which finds the row and tickets cleared."""
+    cfg = P.CONFIGS[name]
+    desc = cfg.desc(n_blocks=1, H=H, W=W)
+    blob, offs = P.synth_weights(desc, seed=9, routing=cfg.routing)
+    engine.load_weights(desc, blob, offs)
+    T, d, N = H * W, cfg.dim, cfg.n_experts
+    n = batch * T
+    x = P.synth_features(cfg, batch=batch, H=H, W=W, seed=10).reshape(-1)
+    feats, aux = device_arena(2 * x.nbytes), device_arena(P.aux_elems(N, n) * 4)
+    hip.upload(feats.ptr, x)
+    pa = engine.attn_push(0, 0, n * d, H, W)
+    for call in ("attn_route", "router", "attn_route", "router"):
+        print(f"[dispatch] {name} {H}x{W} batch {batch} {call}", flush=True)
+        hip.memset(aux.ptr, 0xFF, P.aux_elems(N, n) * 4)
+        pr = engine.router_push(0, T, n * d, 0, n, n + N)
+        rc = engine.attn_route(pa, pr, feats.ptr, aux.ptr, batch) if call == "attn_route" else \
+            engine.router(pr, feats.ptr, aux.ptr, batch)
+        assert rc == 0, engine.error()
+        hip.sync()
+        host = hip.download(np.empty(n + N, np.int32), aux.ptr)
+        assert (host[n:] == np.bincount(host[:n], minlength=N)).all()
