@@ -5,11 +5,14 @@
  * Kernels (extern "C" names, one per stage and supported shape):
  *   prism_attn_d{256,128}[_w8]                     attention stage (4 or 8 waves)
  *   prism_attn_d{256,128}[_w8]_r{1..4}             attention + fused routing
+ *   prism_attn_d{256,128}[_w8]_ffn                 a dense block in one launch
+ *   prism_chain_d{256,128}[_w8]                    every block of a dense chain in one launch
  *   prism_router_d{256,128}_n{1..4}                router + counting sort
  *   prism_expert_d{256,128}_bm64[_w8], _d256_bm{128,96}  grouped expert FFN
  *   prism_project_{up,down}_d{256,128}             projection adapters (128 <-> dim)
- *   prism_codec_enc{0..3}, prism_codec_dec{3,2}    conv encoder / fused decoder stages
- *   prism_codec_enc01, prism_codec_dec21_out       the stages fused in the frame
+ *   prism_codec_enc{0,1}, prism_codec_dec2         conv encoder / fused decoder stages
+ *   prism_codec_enc01, prism_codec_dec21_out       the same, fused in the frame (persistent)
+ *   prism_codec_enc{2,3}, prism_codec_dec3         stages and frame alike (persistent)
  *   prism_codec_dec1_out                           dec1 + output conv + PixelShuffle + sigmoid
  *   prism_zero_i32                                 clears routing counters
  */
