@@ -625,15 +625,17 @@ int enqueue_experts(prism_ctx* c, const DevBlock& k, const uint16_t* in, uint16_
                      : launch(c, c->f_expert_wide, (unsigned)tiles_of(128), a, s, 256u);
     const int64_t tiles = tiles_of(64);
     /* at most one tile per CU: 8 waves per tile halve each wave's weight
-     * stream; otherwise 4 waves x 2 tiles per CU. 64 experts alone on the GPU,
-     * 320 and 448 tiles: 20.9 and 21.7 us on 8 waves (a round of 256 and one
-     * of the rest), 18.6 and 19.6 us on 4. Beside the other sub-chain's
+     * stream; otherwise 4 waves x 2 tiles per CU. Alone on the GPU what counts
+     * is the tiles that hold tokens, about half a tile per expert more than
+     * n / 64 (the rest of the grid ends at once): n / 64 = 246, 16 experts
+     * (254 tiles) 10.2 us on 8 waves, 11.1 on 4; 250 (258) 16.7 and 14.8; 64
+     * experts 220 (252) 10.8 and 11.4; 236 (268) 17.1 and 15.3. Beside the other sub-chain's
      * attention a small second round costs less than slower tiles: a chain
      * with launches of 280 tiles 696 us on 8 waves, 770 on 4; of 296, 745 and
      * 789; of 320, 816 and 832 (or 807 and 789); of 352, 891 and 855. d128
      * tiles leave room for two 8-wave workgroups per CU. */
-    const int64_t w8_tiles = D == 256 ? (stage ? CU_COUNT : CU_COUNT * 5 / 4) : 2 * CU_COUNT - 1;
-    const int w8 = tiles <= w8_tiles ? 1 : 0;
+    const int64_t filled = (n + 63) / 64 + (counts ? N / 2 : 0);
+    const int w8 = D == 256 ? (stage ? filled <= CU_COUNT : tiles <= CU_COUNT * 5 / 4) : tiles < 2 * CU_COUNT;
     return launch(c, c->f_expert[dim_index(D)][w8], (unsigned)tiles, a, s, w8 ? 512u : 256u);
 }
 

@@ -107,3 +107,29 @@ def test_stage_counts_by_the_last_workgroup(hip, engine, device_arena, name, H, 
         hip.sync()
         host = hip.download(np.empty(n + N, np.int32), aux.ptr)
         assert (host[n:] == np.bincount(host[:n], minlength=N)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,W", [("moe16", 248), ("moe16", 249), ("moe64", 224), ("moe64", 225)])
+def test_expert_stage_at_the_edge_of_one_round(hip, engine, device_arena, name, W):
+    """n / 64 + n_experts / 2 = 256 tiles (8 waves) and 257 (4 waves): a frame's
+    rows are the same bits alone and in a batch of two (4 waves)."""
+    H, d = 64, P.CONFIGS[name].dim
+    cfg = P.CONFIGS[name]
+    desc = cfg.desc(n_blocks=1, H=H, W=W)
+    blob, offs = P.synth_weights(desc, seed=11, routing=cfg.routing)
+    engine.load_weights(desc, blob, offs)
+    T, N = H * W, cfg.n_experts
+    x = P.synth_features(cfg, batch=2, H=H, W=W, seed=12).reshape(-1)
+    feats, aux = device_arena(2 * x.nbytes), device_arena(P.aux_elems(N, 2 * T) * 4)
+    ys = []
+    for batch in (1, 2):
+        n = batch * T
+        hip.upload(feats.ptr, x)
+        print(f"[dispatch] experts {name} {H}x{W} batch {batch}", flush=True)
+        assert engine.router(engine.router_push(0, T, 0, 0, n, n + N), feats.ptr, aux.ptr, batch) == 0, engine.error()
+        push = engine.expert_push(0, T, 0, 2 * T * d, 0, n, n + N)
+        assert engine.experts(push, feats.ptr, aux.ptr, batch) == 0, engine.error()
+        hip.sync()
+        ys.append(hip.download(np.empty(T * d, np.uint16), feats.ptr + x.nbytes))
+    assert (ys[0] == ys[1]).all()
