@@ -165,17 +165,26 @@ def chain_launches(eng, dx, dy, batch, stream, reps=5):
     return statistics.median(a), statistics.median(e), ga, ge
 
 
-def sub_chains(cfg, batch):
-    """Parallel sub-chains of the engine's chain: two for a batch of more than
-    192 windows (MoE blocks) or 512 (dense)."""
+def w8(d, windows):
+    """The engine's attention runs as 8-wave workgroups for this many windows."""
+    return "_w8" if windows < (257 if d == 256 else 512) else ""
+
+
+def attn_launch(cfg, batch, grid):
+    """What an attention launch of `grid` windows is in the engine's chain of
+    `batch` frames: its kernel, the blocks it runs and the chain's parallel
+    sub-chains. A dense chain that stays together is one launch for all blocks."""
     windows = ((cfg.W + 7) // 8) * ((cfg.H + 7) // 8) * batch
-    return min(2, batch) if windows > (192 if cfg.n_experts > 1 else 512) else 1
-
-
-def w8(d, workgroups):
-    """The engine's attention runs as 8-wave workgroups for this many windows
-    (over a dense chain's sub-chains)."""
-    return "_w8" if workgroups < (257 if d == 256 else 512) else ""
+    subs = round(windows / grid)
+    moe = cfg.n_experts > 1
+    whole = not moe and subs == 1 and cfg.n_blocks > 1
+    name = f"prism_{'chain' if whole else 'attn'}_d{cfg.dim}"
+    name += w8(cfg.dim, grid if moe else windows)
+    if moe:
+        name += f"_r{(cfg.n_experts + 15) // 16}"
+    elif not whole:
+        name += "_ffn"
+    return name, cfg.n_blocks if whole else 1, subs
 
 
 def expert_kernel(d, tokens, n_experts):
@@ -293,19 +302,18 @@ def config_section(hip, name, batch, steps, stream):
     finally:
         eng.close()
     flops_frame = cfg.flops_per_token_block() * T * cfg.n_blocks
-    S = sub_chains(cfg, batch)
+    kern, nb, S = attn_launch(cfg, batch, ga)
     tok_launch = batch * T // S
     a_flops = (attn_flops_per_token(cfg) + router_flops_per_token(cfg)) * tok_launch
     e_flops = 2 * 2 * d * d * tok_launch
-    fused = ge == 0  # dense d128 blocks: the FFN runs inside the attention launch
+    fused = ge == 0  # dense blocks: the FFN runs inside the attention launch
     if fused:
-        a_flops += e_flops
-    kern = f"prism_attn_d{d}" + w8(d, ga if cfg.n_experts > 1 else ga * S) + (f"_r{(cfg.n_experts + 15) // 16}" if cfg.n_experts > 1 else "") + ("_ffn" if fused else "")
+        a_flops = nb * (a_flops + e_flops)
     return {"batch": batch, "ms_per_step": round(ms_b, 5), "frames_per_s": round(batch / (ms_b * 1e-3), 2),
             "mfma_frac": round(flops_frame * batch / (ms_b * 1e-3) / MFMA_F16_PEAK, 4),
             "batch1_us_per_frame": round(ms_1 * 1e3, 2),
             "batch1_mfma_frac": round(flops_frame / (ms_1 * 1e-3) / MFMA_F16_PEAK, 4),
-            "roofline": {"kernel": kern, "grid": ga, "avg_launch_ms": round(ta, 5),
+            "roofline": {"kernel": kern, "grid": ga, "blocks_per_launch": nb, "avg_launch_ms": round(ta, 5),
                          "frac": round(a_flops / (ta * 1e-3) / MFMA_F16_PEAK, 4),
                          "expert_grid": ge, "expert_avg_launch_ms": None if fused else round(te, 5),
                          "expert_frac": None if fused else round(e_flops / (te * 1e-3) / MFMA_F16_PEAK, 4)},
@@ -406,15 +414,13 @@ def main():
     # one after another with HIP events between them
     log("[bench] chain launches")
     c_attn, c_exp, c_ga, c_ge = chain_launches(eng, dx, dy, B, stream)
-    S = sub_chains(cfg, B)
+    c_kname, c_nb, S = attn_launch(cfg, B, c_ga)
     tok_launch = n // S
     c_attn_flops = (attn_flops_per_token(cfg) + router_flops_per_token(cfg)) * tok_launch
     c_exp_flops = 2 * 2 * d * d * tok_launch
-    c_fused = c_ge == 0  # dense d128 blocks: the FFN runs inside the attention launch
+    c_fused = c_ge == 0  # dense blocks: the FFN runs inside the attention launch
     if c_fused:
-        c_attn_flops, c_exp_flops = c_attn_flops + c_exp_flops, 0
-    c_kname = (f"prism_attn_d{d}" + w8(d, c_ga if moe else c_ga * S) + (f"_r{(N + 15) // 16}" if moe else "")
-               + ("_ffn" if c_fused else ""))
+        c_attn_flops, c_exp_flops = c_nb * (c_attn_flops + c_exp_flops), 0
     c_ename = None if c_fused else expert_kernel(d, tok_launch, N)
     c_traffic, c_traffic_src = measured_traffic(c_kname, c_ga) if cfg.name == "moe64" else (None, None)
     c_etraffic, _ = measured_traffic(c_ename, c_ge) if cfg.name == "moe64" else (None, None)
@@ -500,7 +506,7 @@ def main():
                      "timed": f"the batch-{B} chain's own attention launches ({c_ga} workgroups, {tok_launch} tokens "
                               "each), run one after another by prism_chain_launch_times: HIP events between "
                               "launches on the launch stream, median over 5 chains of the mean over the chain's "
-                              f"{cfg.n_blocks * S} launches",
+                              f"{cfg.n_blocks // c_nb * S} launches",
                      "chain_launches": {
                          "attention": {"kernel": c_kname, "grid": c_ga, "flops": c_attn_flops,
                                        "avg_launch_ms": round(c_attn, 5),

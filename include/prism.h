@@ -253,9 +253,8 @@ int prism_forward_noalloc(prism_ctx* ctx, const void* in, void* out, int32_t bat
  * (expert_ms), and the workgroup count of each (the first launch of each
  * kind). A dense block runs its FFN inside its attention launch, so a dense
  * model reports expert_ms = 0 and expert_grid = 0; where prism_forward takes a
- * dense chain through all its blocks in one launch, the blocks are launched
- * one by one here (the same output). `out` receives the
- * chain's output, as from prism_forward. */
+ * dense chain through all its blocks in one launch, attn_ms is that launch's
+ * duration. `out` receives the chain's output, as from prism_forward. */
 int prism_chain_launch_times(prism_ctx* ctx, const void* in, void* out, int32_t batch, void* stream,
                              float* attn_ms, float* expert_ms, int32_t* attn_grid, int32_t* expert_grid);
 

@@ -12,7 +12,6 @@
  */
 #include <hip/hip_runtime.h>
 
-#include <algorithm>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -31,10 +30,6 @@ const int kOutRes[N_STAGES] = {0, 1, 2, 3, 2, 1, 0}; /* of the output map (dec1:
 const int kInCh[N_STAGES] = {9, 32, 64, 128, 128, 128, 64};
 const int kSkipCh[N_STAGES] = {0, 0, 0, 0, 128, 64, 32};
 const int kOutCh[N_STAGES] = {32, 64, 128, 128, 128, 64, 12}; /* dec1: 12 channels = 3 planes x 2x2 */
-
-/* workgroups of the persistent codec launches the GPU holds at once */
-constexpr int CODEC_DEC3_SLOTS = 3 * CU_COUNT, CODEC_DEC21_SLOTS = 3 * CU_COUNT, CODEC_ENC01_SLOTS = 2 * CU_COUNT,
-              CODEC_ENC2_SLOTS = 2 * CU_COUNT, CODEC_ENC3_SLOTS = 2 * CU_COUNT;
 
 bool aligned16(const void* p) { return ((uintptr_t)p & 15) == 0; }
 
@@ -63,14 +58,6 @@ CodecArgs stage_args(const prism_ctx* c, int st, const uint16_t* in, const uint1
     return a;
 }
 
-/* Grid of a persistent decoder launch: `slots` workgroups at once, every one
- * the same number of the launch's blocks (or one fewer), so no workgroup is
- * left with a block of its own at the end. */
-unsigned even_grid(int64_t blocks, int slots) {
-    const int64_t each = (blocks + slots - 1) / slots;
-    return (unsigned)((blocks + each - 1) / each);
-}
-
 /* Blocks of rows x cols pixels of a w x h map. */
 int blocks_of(int w, int h, int rows, int cols) { return ((w + cols - 1) / cols) * ((h + rows - 1) / rows); }
 
@@ -94,9 +81,11 @@ int launch_blocks(prism_ctx* c, hipFunction_t f, const char* what, int per_frame
 int launch_stage(prism_ctx* c, int st, const uint16_t* in, const uint16_t* skip, uint16_t* out, int batch,
                  hipStream_t s) {
     CodecArgs a = stage_args(c, st, in, skip, out);
-    if (st == ST_ENC2)
-        return launch_blocks(c, c->f_codec[st], "enc2", blocks_of(a.out_w, a.out_h, CODEC_ENC2_ROWS, CODEC_ENC2_COLS), batch,
-                             CODEC_ENC2_SLOTS, true, 512, s, a);
+    if (st == ST_ENC2) {
+        const int per_frame = blocks_of(a.out_w, a.out_h, CODEC_ENC2_ROWS, CODEC_ENC2_COLS);
+        return launch_blocks(c, c->f_codec[st], "enc2", per_frame, batch, codec_enc2_slots((int64_t)per_frame * batch), true,
+                             512, s, a);
+    }
     if (st == ST_ENC3)
         return launch_blocks(c, c->f_codec[st], "enc3", blocks_of(a.out_w, a.out_h, CODEC_ENC3_ROWS, CODEC_ENC3_COLS), batch,
                              CODEC_ENC3_SLOTS, true, 512, s, a);

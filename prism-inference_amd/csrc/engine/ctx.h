@@ -11,6 +11,7 @@
 
 #include "../kernel_args.h"
 #include "prism.h"
+#include "rules.h"
 
 namespace prism {
 
@@ -32,24 +33,14 @@ struct DevBlock {
 
 }  // namespace prism
 
+using prism::CHAIN_SPLIT;
+using prism::CU_COUNT;
 using prism::DevBlock;
 
 /* The chain's per-expert counters sit 256 bytes apart: every workgroup of a
  * routed attention launch adds to them, and counters sharing a cache line
  * would serialise those atomics in one memory channel. */
 static constexpr int CHAIN_COUNT_STRIDE = 64;
-/* Compute units of an MI355X. */
-static constexpr int CU_COUNT = 256;
-/* The chain of a batch with more than CHAIN_SPLIT_ROUTED (MoE blocks) or
- * CHAIN_SPLIT_DENSE windows (see chain_split) runs as up to CHAIN_SPLIT
- * independent sub-chains of whole frames, on their own streams
- * (parallel branches of the hipGraph): windows and tokens never interact
- * across frames, and one sub-chain's expert launches overlap another's
- * attention launches and the tails of both. */
-static constexpr int CHAIN_SPLIT = 2;
-static constexpr int CHAIN_SPLIT_ROUTED = CU_COUNT * 3 / 4;
-static constexpr int CHAIN_SPLIT_DENSE = 2 * CU_COUNT;
-static_assert(CHAIN_SPLIT >= 1 && CHAIN_SPLIT <= 4, "sub-chain streams");
 /* d256 expert launches of at least this many 128-token tiles (two per CU)
  * use the 128-token kernel: each streamed weight fragment then feeds twice
  * the tokens. Smaller grids keep 64-token tiles (8 waves up to CU_COUNT tiles).
@@ -66,13 +57,6 @@ static constexpr int EXPERT_WIDE_MIN_TILES = 512;
  * to the next instead of the whole cyclic stream missing (prism_load_weights
  * sets wnt_blocks). */
 static constexpr int64_t WEIGHT_CACHE_KEEP = 224ll << 20;
-/* Workgroups of a projection stage launch (persistent, 64-token tiles in a
- * loop, two per CU); at d256 up to PROJ_SINGLE_MAX tiles go one to a
- * workgroup. Both d256 launches, 765 tiles: 19.1 us on 512 workgroups, 18.3 on
- * 765; 2,040 tiles: 41.5 on 512, 43.7 on 768. */
-static constexpr int PROJ_GRID_MAX = 512;
-static constexpr int PROJ_SINGLE_MAX = 768;
-
 /* Attention keys all 64 slots of a window. The reference keys the first
  * min(64, n_tokens) slots in slot order (split2_qkv_attn_d256.comp.glsl:33,60),
  * which differs only for frames of fewer than 64 tokens: those are refused. */

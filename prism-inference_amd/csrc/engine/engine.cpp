@@ -538,16 +538,7 @@ int enqueue_attn(prism_ctx* c, const DevBlock& k, const uint16_t* in, uint16_t* 
     }
     const int64_t grid = (int64_t)a.windows_per_frame * batch;
     if (grid <= 0 || grid > 0x7fffffff) return fail(c, PRISM_ERR_INVALID, "attention grid %lld out of range", (long long)grid);
-    /* Windows that fit the CUs as 8-wave workgroups (a head per wave) take
-     * those, which shortens each window's serial path; more of them go as
-     * 4-wave workgroups, two per CU (three at d128). A d256 8-wave workgroup fills its CU's registers,
-     * so window 257 starts a second round: routed launches of 270, 405 and
-     * 510 windows take 28.6, 32.6 and 35 us on 8 waves, 23.6, 27.5 and 30.7
-     * on 4, and one of 135 takes 16.8 us on 8. Two d128 ones share a CU (270
-     * windows 13.0 us either way, 405 16.3 and 16.0). With par > 1 the
-     * launches' windows count together (two dense launches of 256 at once: 162
-     * us a four-block chain on 8 waves, 134 on 4). */
-    const int w8 = grid * par < (D == 256 ? CU_COUNT + 1 : 2 * CU_COUNT) ? 1 : 0;
+    const int w8 = attn_w8(D, grid, par) ? 1 : 0;
     if (blocks > 1) {
         const DevBlock* const kb = &k;
         a.n_blocks = blocks;
@@ -624,18 +615,7 @@ int enqueue_experts(prism_ctx* c, const DevBlock& k, const uint16_t* in, uint16_
         return stage ? launch(c, c->f_expert_wide96, (unsigned)tiles_of(96), a, s, 256u)
                      : launch(c, c->f_expert_wide, (unsigned)tiles_of(128), a, s, 256u);
     const int64_t tiles = tiles_of(64);
-    /* at most one tile per CU: 8 waves per tile halve each wave's weight
-     * stream; otherwise 4 waves x 2 tiles per CU. Alone on the GPU what counts
-     * is the tiles that hold tokens, about half a tile per expert more than
-     * n / 64 (the rest of the grid ends at once): n / 64 = 246, 16 experts
-     * (254 tiles) 10.2 us on 8 waves, 11.1 on 4; 250 (258) 16.7 and 14.8; 64
-     * experts 220 (252) 10.8 and 11.4; 236 (268) 17.1 and 15.3. Beside the other sub-chain's
-     * attention a small second round costs less than slower tiles: a chain
-     * with launches of 280 tiles 696 us on 8 waves, 770 on 4; of 296, 745 and
-     * 789; of 320, 816 and 832 (or 807 and 789); of 352, 891 and 855. d128
-     * tiles leave room for two 8-wave workgroups per CU. */
-    const int64_t filled = (n + 63) / 64 + (counts ? N / 2 : 0);
-    const int w8 = D == 256 ? (stage ? filled <= CU_COUNT : tiles <= CU_COUNT * 5 / 4) : tiles < 2 * CU_COUNT;
+    const int w8 = expert_w8(D, tiles, n, counts ? N : 0, stage) ? 1 : 0;
     return launch(c, c->f_expert[dim_index(D)][w8], (unsigned)tiles, a, s, w8 ? 512u : 256u);
 }
 
@@ -649,11 +629,9 @@ int enqueue_project(prism_ctx* c, bool up, const uint16_t* in, uint16_t* out, in
     a.n_tokens = n;
     const int64_t tiles = (n + 63) / 64;
     if (tiles <= 0 || tiles > 0x7fffffff) return fail(c, PRISM_ERR_INVALID, "projection tiles %lld out of range", (long long)tiles);
-    /* persistent workgroups looping over 64-token tiles; at d256 a tile each
-     * while they are few (ctx.h) */
-    const bool d256 = c->desc.dim == 256;
-    const int64_t grid = d256 && tiles <= PROJ_SINGLE_MAX ? tiles : std::min<int64_t>(tiles, PROJ_GRID_MAX);
-    return launch(c, c->f_proj[dim_index(c->desc.dim)][up ? 0 : 1], (unsigned)grid, a, s, d256 ? 512u : 256u);
+    /* persistent workgroups looping over 64-token tiles */
+    const int D = c->desc.dim;
+    return launch(c, c->f_proj[dim_index(D)][up ? 0 : 1], (unsigned)project_grid(D, tiles), a, s, D == 256 ? 512u : 256u);
 }
 
 /* which: 0 = attention (qkv_w), 1 = router (router_w), 2 = experts (exp_w1) */
@@ -918,34 +896,6 @@ static int ensure_workspace(prism_ctx* c, int batch, bool io = false) {
  * A large batch runs as sub-chains (own counter rows, own bucket region,
  * disjoint frames of every buffer). */
 
-/* Sub-chains of a forward. A routed block's two launches leave CUs idle in
- * turn (the attention's while its last windows finish, the experts' while
- * they wait for weights), so the frames of a batch go in halves as soon as
- * one half's attention launch no longer fits beside the other's experts for
- * free: 16 blocks, one chain against two: 160 windows 411 and 418 us, 192
- * 442 and 438, 256 578 and 509 (64 experts), 270 641 and 504, 288 684 and
- * 539, 504 859 and 814. A dense block is one launch: its frames stay together
- * while they fit one round of the 4-wave kernels (two workgroups per CU; four
- * blocks, 256 windows 83 and 91 us, d128 512 windows 61 and 74; 540 windows
- * 170 and 150). */
-static int chain_split(const prism_model_desc& d, int batch) {
-    const int64_t windows = (int64_t)((d.spatial_w + 7) / 8) * ((d.spatial_h + 7) / 8) * batch;
-    return windows > (d.n_experts > 1 ? CHAIN_SPLIT_ROUTED : CHAIN_SPLIT_DENSE) ? std::min(CHAIN_SPLIT, batch) : 1;
-}
-
-/* A dense chain's windows meet no others in any block, so one launch can take
- * each through all of them with its rows in LDS: no launch, row load or store
- * between the blocks. At d256 while the windows fit one round of workgroups
- * (two 4-wave ones per CU): 12 blocks of 135, 270 and 405 windows 195 -> 151,
- * 267 -> 229 and 339 -> 300 us; of 540 windows, whose second round is nearly
- * empty for all 12 blocks, 393 and 430; of 1,080, 699 and 739. At d128, whose
- * windows are short, always: 4 blocks of 135, 540, 1,080 and 2,160 windows
- * 38 -> 31, 72 -> 57, 104 -> 98 and 182 -> 172 us. */
-static bool dense_one_launch(const prism_model_desc& d, int batch) {
-    const int64_t windows = (int64_t)((d.spatial_w + 7) / 8) * ((d.spatial_h + 7) / 8) * batch;
-    return d.n_experts == 1 && (d.dim == 128 || windows <= 2 * CU_COUNT);
-}
-
 /* Sub-chain j: frames [f0, f0 + nf) through every block, in -> out (this
  * sub-chain's frames). adapted: in and out hold 128-channel rows; block 0's
  * attention runs the up-projection in its prologue and the last block's
@@ -973,11 +923,11 @@ static int timer_mark(prism_ctx* c, ChainTimer* tm, int kind, hipStream_t s) {
     return PRISM_OK;
 }
 
-static int enqueue_subchain(prism_ctx* c, const ChainWs& ws, int S, int j, int f0, int nf, const uint16_t* in,
+static int enqueue_subchain(prism_ctx* c, const ChainWs& ws, const ChainPlan& plan, int j, int f0, int nf, const uint16_t* in,
                             uint16_t* out, hipStream_t s, bool adapted = false, ChainTimer* tm = nullptr) {
     const int NB = c->desc.n_blocks, H = c->desc.spatial_h, W = c->desc.spatial_w, D = c->desc.dim;
     const int N = c->desc.n_experts;
-    const bool moe = N > 1;
+    const bool moe = N > 1, one_launch = plan.one_launch;
     const int64_t T = (int64_t)H * W, n = (int64_t)nf * T, t0 = (int64_t)f0 * T, n_all = ws.n;
     const size_t row = (size_t)N * CHAIN_COUNT_STRIDE;
     int32_t* counts0 = ws.counts + (size_t)j * NB * row;
@@ -991,11 +941,12 @@ static int enqueue_subchain(prism_ctx* c, const ChainWs& ws, int S, int j, int f
     }
     const uint16_t* src = in;
     int b0 = 0;
-    if (!moe && !tm && S == 1 && dense_one_launch(c->desc, nf)) { /* every block but the one the down-projection follows */
+    if (one_launch) { /* every block but the one the down-projection follows */
         b0 = adapted ? NB - 1 : NB;
         if (b0 > 1) {
             uint16_t* dst = b0 == NB ? out : scratch;
-            const int rc = enqueue_attn(c, c->blocks[0], src, dst, H, W, nf, s, nullptr, adapted, true, 1, b0);
+            int rc = enqueue_attn(c, c->blocks[0], src, dst, H, W, nf, s, nullptr, adapted, true, 1, b0);
+            if (!rc) rc = timer_mark(c, tm, 0, s);
             if (rc) return rc;
             src = dst;
         } else {
@@ -1018,11 +969,11 @@ static int enqueue_subchain(prism_ctx* c, const ChainWs& ws, int S, int j, int f
             if (!rc) rc = timer_mark(c, tm, 1, s);
             if (rc) return rc;
         } else if (!last) { /* one launch: attention + the FFN */
-            int rc = enqueue_attn(c, k, src, dst, H, W, nf, s, nullptr, first, true, S);
+            int rc = enqueue_attn(c, k, src, dst, H, W, nf, s, nullptr, first, true, plan.split);
             if (!rc) rc = timer_mark(c, tm, 0, s);
             if (rc) return rc;
         } else {
-            int rc = enqueue_attn(c, k, src, attn, H, W, nf, s, nullptr, first, false, S);
+            int rc = enqueue_attn(c, k, src, attn, H, W, nf, s, nullptr, first, false, plan.split);
             if (!rc) rc = timer_mark(c, tm, 0, s);
             if (!rc) rc = enqueue_experts(c, k, attn, dst, nullptr, nullptr, n, s, 1, last);
             if (!rc) rc = timer_mark(c, tm, 1, s);
@@ -1039,8 +990,9 @@ static int enqueue_forward_impl(prism_ctx* c, const ChainWs& ws, const uint16_t*
     const int64_t D = adapted ? c->aoffs.in_dim : c->desc.dim; /* channels of in and out */
     c->fwd_tokens = (int64_t)batch * T;
     c->fwd_assign = ws.assign;
-    const int S = dense_one_launch(c->desc, batch) ? 1 : chain_split(c->desc, batch);
-    if (S == 1) return enqueue_subchain(c, ws, 1, 0, 0, batch, in, out, s, adapted);
+    const ChainPlan plan = chain_plan(c->desc, batch);
+    const int S = plan.split;
+    if (S == 1) return enqueue_subchain(c, ws, plan, 0, 0, batch, in, out, s, adapted);
     /* fork: sub-chain j > 0 on sub_stream[j-1], sub-chain 0 on s, then join */
     HIP_TRY(c, hipEventRecord(c->ev_fork, s));
     int rc = PRISM_OK;
@@ -1048,7 +1000,7 @@ static int enqueue_forward_impl(prism_ctx* c, const ChainWs& ws, const uint16_t*
         const int f0 = (int)((int64_t)batch * j / S), f1 = (int)((int64_t)batch * (j + 1) / S);
         hipStream_t sj = j ? c->sub_stream[j - 1] : s;
         if (j) HIP_TRY(c, hipStreamWaitEvent(sj, c->ev_fork, 0));
-        const int r = enqueue_subchain(c, ws, S, j, f0, f1 - f0, in + f0 * T * D, out + f0 * T * D, sj, adapted);
+        const int r = enqueue_subchain(c, ws, plan, j, f0, f1 - f0, in + f0 * T * D, out + f0 * T * D, sj, adapted);
         if (!rc) rc = r;
         if (j) HIP_TRY(c, hipEventRecord(c->ev_join[j - 1], sj));
     }
@@ -1204,8 +1156,9 @@ extern "C" int prism_chain_launch_times(prism_ctx* c, const void* in, void* out,
     ws.n = (int64_t)batch * T;
     c->fwd_tokens = ws.n;
     c->fwd_assign = ws.assign;
-    /* the sub-chains of prism_forward, one after another on one stream */
-    const int S = chain_split(c->desc, batch);
+    /* prism_forward's launches, one sub-chain after another on one stream */
+    const ChainPlan plan = chain_plan(c->desc, batch);
+    const int S = plan.split;
     ChainTimer tm;
     tm.ev.assign((size_t)2 * c->desc.n_blocks * S + 1, nullptr);
     for (auto& e : tm.ev) {
@@ -1221,7 +1174,7 @@ extern "C" int prism_chain_launch_times(prism_ctx* c, const void* in, void* out,
     rc = timer_mark(c, &tm, -1, s);
     for (int j = 0; j < S && !rc; ++j) {
         const int f0 = (int)((int64_t)batch * j / S), f1 = (int)((int64_t)batch * (j + 1) / S);
-        rc = enqueue_subchain(c, ws, S, j, f0, f1 - f0, src + f0 * T * D, dst + f0 * T * D, s, false, &tm);
+        rc = enqueue_subchain(c, ws, plan, j, f0, f1 - f0, src + f0 * T * D, dst + f0 * T * D, s, false, &tm);
     }
     if (rc) c->counts_dirty = true; /* launched part of the chain */
     double sum[2] = {0, 0};

@@ -1,0 +1,122 @@
+/* rules.h - which kernel, how many waves and how many workgroups a call gets,
+ * as functions of sizes alone (no HIP). Host plain C++. */
+#ifndef PRISM_RULES_H
+#define PRISM_RULES_H
+
+#include <algorithm>
+#include <cstdint>
+
+#include "prism.h"
+
+namespace prism {
+
+/* Compute units of an MI355X. */
+constexpr int CU_COUNT = 256;
+
+/* ---- block chain */
+
+/* The chain of a batch with more than CHAIN_SPLIT_ROUTED (MoE blocks) or
+ * CHAIN_SPLIT_DENSE windows (see chain_plan) runs as up to CHAIN_SPLIT
+ * independent sub-chains of whole frames, on their own streams
+ * (parallel branches of the hipGraph): windows and tokens never interact
+ * across frames, and one sub-chain's expert launches overlap another's
+ * attention launches and the tails of both. */
+constexpr int CHAIN_SPLIT = 2;
+constexpr int CHAIN_SPLIT_ROUTED = CU_COUNT * 3 / 4;
+constexpr int CHAIN_SPLIT_DENSE = 2 * CU_COUNT;
+static_assert(CHAIN_SPLIT >= 1 && CHAIN_SPLIT <= 4, "sub-chain streams");
+
+/* How a forward's blocks are launched. */
+struct ChainPlan {
+    int split;       /* sub-chains */
+    bool one_launch; /* a dense chain: every block in one launch */
+};
+
+/* Sub-chains. A routed block's two launches leave CUs idle in
+ * turn (the attention's while its last windows finish, the experts' while
+ * they wait for weights), so the frames of a batch go in halves as soon as
+ * one half's attention launch no longer fits beside the other's experts for
+ * free: 16 blocks, one chain against two: 160 windows 411 and 418 us, 192
+ * 442 and 438, 256 578 and 509 (64 experts), 270 641 and 504, 288 684 and
+ * 539, 504 859 and 814. A dense block is one launch: its frames stay together
+ * while they fit one round of the 4-wave kernels (two workgroups per CU; four
+ * blocks, 256 windows 83 and 91 us, d128 512 windows 61 and 74; 540 windows
+ * 170 and 150).
+ *
+ * One launch. A dense chain's windows meet no others in any block, so one launch can take
+ * each through all of them with its rows in LDS: no launch, row load or store
+ * between the blocks. At d256 while the windows fit one round of workgroups
+ * (two 4-wave ones per CU): 12 blocks of 135, 270 and 405 windows 195 -> 151,
+ * 267 -> 229 and 339 -> 300 us; of 540 windows, whose second round is nearly
+ * empty for all 12 blocks, 393 and 430; of 1,080, 699 and 739. At d128, whose
+ * windows are short, always: 4 blocks of 135, 540, 1,080 and 2,160 windows
+ * 38 -> 31, 72 -> 57, 104 -> 98 and 182 -> 172 us. */
+inline ChainPlan chain_plan(const prism_model_desc& d, int batch) {
+    const int64_t windows = (int64_t)((d.spatial_w + 7) / 8) * ((d.spatial_h + 7) / 8) * batch;
+    if (d.n_experts > 1) return {windows > CHAIN_SPLIT_ROUTED ? std::min(CHAIN_SPLIT, batch) : 1, false};
+    if (d.dim == 128 || windows <= 2 * CU_COUNT) return {1, true};
+    return {windows > CHAIN_SPLIT_DENSE ? std::min(CHAIN_SPLIT, batch) : 1, false};
+}
+
+/* Attention: 8 waves (a workgroup per CU at d256)? Windows that fit the CUs as
+ * 8-wave workgroups (a head per wave) take those, which shortens each window's
+ * serial path; more of them go as 4-wave workgroups, two per CU (three at
+ * d128). A d256 8-wave workgroup fills its CU's registers, so window 257
+ * starts a second round: routed launches of 270, 405 and 510 windows take
+ * 28.6, 32.6 and 35 us on 8 waves, 23.6, 27.5 and 30.7 on 4, and one of 135
+ * takes 16.8 us on 8. Two d128 ones share a CU (270 windows 13.0 us either
+ * way, 405 16.3 and 16.0). par: attention launches of about this size that run
+ * at the same time (a dense chain's sub-chains; a routed one's run beside the
+ * other's experts); their windows count together (two dense launches of 256 at
+ * once: 162 us a four-block chain on 8 waves, 134 on 4). */
+inline bool attn_w8(int dim, int64_t windows, int par) {
+    return windows * par < (dim == 256 ? CU_COUNT + 1 : 2 * CU_COUNT);
+}
+
+/* Experts, 64-token tiles: 8 waves? tiles: the launch's grid, n / 64 and a
+ * partial tile per expert; n: its tokens; partial: the experts (0 if dense).
+ * At most one tile per CU: 8 waves per tile halve each wave's weight
+ * stream; otherwise 4 waves x 2 tiles per CU. Alone on the GPU what counts
+ * is the tiles that hold tokens, about half a tile per expert more than
+ * n / 64 (the rest of the grid ends at once): n / 64 = 246, 16 experts
+ * (254 tiles) 10.2 us on 8 waves, 11.1 on 4; 250 (258) 16.7 and 14.8; 64
+ * experts 220 (252) 10.8 and 11.4; 236 (268) 17.1 and 15.3. Beside the other sub-chain's
+ * attention a small second round costs less than slower tiles: a chain
+ * with launches of 280 tiles 696 us on 8 waves, 770 on 4; of 296, 745 and
+ * 789; of 320, 816 and 832 (or 807 and 789); of 352, 891 and 855. d128
+ * tiles leave room for two 8-wave workgroups per CU. */
+inline bool expert_w8(int dim, int64_t tiles, int64_t n, int partial, bool stage) {
+    if (dim != 256) return tiles < 2 * CU_COUNT;
+    return stage ? (n + 63) / 64 + partial / 2 <= CU_COUNT : tiles <= CU_COUNT * 5 / 4;
+}
+
+/* ---- projection stages */
+
+/* Workgroups of a projection stage launch (persistent, 64-token tiles in a
+ * loop, two per CU); at d256 up to PROJ_SINGLE_MAX tiles go one to a
+ * workgroup. Both d256 launches, 765 tiles: 19.1 us on 512 workgroups, 18.3 on
+ * 765; 2,040 tiles: 41.5 on 512, 43.7 on 768. */
+constexpr int PROJ_GRID_MAX = 512;
+constexpr int PROJ_SINGLE_MAX = 768;
+inline int64_t project_grid(int dim, int64_t tiles) {
+    return dim == 256 && tiles <= PROJ_SINGLE_MAX ? tiles : std::min<int64_t>(tiles, PROJ_GRID_MAX);
+}
+
+/* ---- codec */
+
+/* workgroups of the persistent codec launches the GPU holds at once */
+constexpr int CODEC_DEC3_SLOTS = 3 * CU_COUNT, CODEC_DEC21_SLOTS = 3 * CU_COUNT, CODEC_ENC01_SLOTS = 2 * CU_COUNT,
+              CODEC_ENC3_SLOTS = 2 * CU_COUNT;
+inline int codec_enc2_slots(int64_t) { return 2 * CU_COUNT; }
+
+/* Grid of a persistent codec launch: `slots` workgroups at once, every one
+ * the same number of the launch's blocks (or one fewer), so no workgroup is
+ * left with a block of its own at the end. */
+inline unsigned even_grid(int64_t blocks, int slots) {
+    const int64_t each = (blocks + slots - 1) / slots;
+    return (unsigned)((blocks + each - 1) / each);
+}
+
+}  // namespace prism
+
+#endif

@@ -1,0 +1,25 @@
+/* The engine's dispatch rules (csrc/engine/rules.h) for ctypes. */
+#include "../prism-inference_amd/csrc/engine/rules.h"
+
+using namespace prism;
+
+static prism_model_desc desc(int dim, int experts, int h, int w) {
+    prism_model_desc d{};
+    d.dim = dim;
+    d.n_experts = experts;
+    d.spatial_h = h;
+    d.spatial_w = w;
+    return d;
+}
+
+extern "C" {
+/* sub-chains, negative where every block runs in one launch */
+int chain(int dim, int experts, int h, int w, int batch) {
+    const ChainPlan p = chain_plan(desc(dim, experts, h, w), batch);
+    return p.one_launch ? -p.split : p.split;
+}
+int attention_waves(int dim, long long windows, int par) { return attn_w8(dim, windows, par) ? 8 : 4; }
+long long projection_grid(int dim, long long tiles) { return project_grid(dim, tiles); }
+int enc2_slots(long long blocks) { return codec_enc2_slots(blocks); }
+unsigned grid_of(long long blocks, int slots) { return even_grid(blocks, slots); }
+}

@@ -1,0 +1,49 @@
+"""Which kernels and grids the engine chooses, by size (csrc/engine/rules.h,
+compiled here into a small library): the edges of each rule."""
+import ctypes as C
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ONE = -1  # every block in one launch
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("rules") / "rules.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__",
+                    "-I", os.path.join(HERE, "..", "include"), os.path.join(HERE, "dispatch_rules.cpp"), "-o", so],
+                   check=True, timeout=120)
+    lib = C.CDLL(so)
+    lib.attention_waves.argtypes = [C.c_int, C.c_longlong, C.c_int]
+    lib.projection_grid.argtypes, lib.projection_grid.restype = [C.c_int, C.c_longlong], C.c_longlong
+    lib.enc2_slots.argtypes = [C.c_longlong]
+    lib.grid_of.argtypes, lib.grid_of.restype = [C.c_longlong, C.c_int], C.c_uint
+    return lib
+
+
+@pytest.mark.parametrize("dim,experts,h,w,batch,plan", [
+    (256, 64, 64, 64, 3, 1), (256, 64, 64, 64, 4, 2),      # 192 | 256 windows
+    (256, 16, 135, 240, 1, 1),                             # one frame never splits
+    (128, 1, 68, 120, 1, ONE), (128, 1, 68, 120, 16, ONE),  # d128: always together
+    (256, 1, 64, 64, 4, ONE),                              # 256 windows
+    (256, 1, 64, 64, 8, ONE), (256, 1, 64, 64, 9, 2),      # 512 | 576
+    (256, 1, 135, 240, 2, 2),
+])
+def test_chain_plan(rules, dim, experts, h, w, batch, plan):
+    assert rules.chain(dim, experts, h, w, batch) == plan
+
+
+def test_attention_waves(rules):
+    assert [rules.attention_waves(256, n, 1) for n in (1, 256, 257)] == [8, 8, 4]
+    assert [rules.attention_waves(128, n, 1) for n in (511, 512)] == [8, 4]
+
+
+@pytest.mark.parametrize("blocks,slots", [(1, 512), (511, 512), (512, 512), (513, 512), (1021, 256), (10**6, 768)])
+def test_every_workgroup_of_a_persistent_launch_has_a_block(rules, blocks, slots):
+    g = rules.grid_of(blocks, slots)
+    each = -(-blocks // g)
+    assert 0 < g <= slots and (each - 1) * g < blocks <= each * g
+    assert each == -(-blocks // slots)
