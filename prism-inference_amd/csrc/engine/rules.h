@@ -107,7 +107,18 @@ inline int64_t project_grid(int dim, int64_t tiles) {
 /* workgroups of the persistent codec launches the GPU holds at once */
 constexpr int CODEC_DEC3_SLOTS = 3 * CU_COUNT, CODEC_DEC21_SLOTS = 3 * CU_COUNT, CODEC_ENC01_SLOTS = 2 * CU_COUNT,
               CODEC_ENC3_SLOTS = 2 * CU_COUNT;
-inline int codec_enc2_slots(int64_t) { return 2 * CU_COUNT; }
+/* enc2 of up to four blocks per CU runs one workgroup per CU. Two of its
+ * workgroups on every CU draw so much that the GPU lowers its clock for
+ * hundreds of microseconds after them: behind an encode of 960x540 (510
+ * blocks) every launch of a chain ran 4 % slower (16 MoE blocks 421 against
+ * 406 us, 2,372 against 2,395 MHz on average), so the frame lost what the
+ * encoder had gained: 466 -> 449 us; the 12-block dense model's 236 -> 224,
+ * two MoE frames 612 -> 603. The encode itself gains too: 960x540 34.7 -> 33.8,
+ * 1280x720 (920 blocks) 54.7 -> 53.4, two of 960x540 (1,020) 56.6 -> 55.5.
+ * Above, two workgroups hide each other's waits: three frames (1,530) 85.5
+ * against 86.4, 1920x1080 (2,040) 108.1 against 109.4, and the frame's chain
+ * is long enough to take no harm (1,052 us either way). */
+inline int codec_enc2_slots(int64_t blocks) { return blocks <= 4 * CU_COUNT ? CU_COUNT : 2 * CU_COUNT; }
 
 /* Grid of a persistent codec launch: `slots` workgroups at once, every one
  * the same number of the launch's blocks (or one fewer), so no workgroup is

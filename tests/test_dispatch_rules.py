@@ -41,6 +41,12 @@ def test_attention_waves(rules):
     assert [rules.attention_waves(128, n, 1) for n in (511, 512)] == [8, 4]
 
 
+@pytest.mark.parametrize("blocks,grid", [(256, 256), (257, 129), (510, 255), (1024, 256), (1025, 342), (2040, 510)])
+def test_enc2_keeps_to_one_workgroup_per_cu(rules, blocks, grid):
+    """Two per CU pull the clock down for the chain that follows."""
+    assert rules.grid_of(blocks, rules.enc2_slots(blocks)) == grid
+
+
 @pytest.mark.parametrize("blocks,slots", [(1, 512), (511, 512), (512, 512), (513, 512), (1021, 256), (10**6, 768)])
 def test_every_workgroup_of_a_persistent_launch_has_a_block(rules, blocks, slots):
     g = rules.grid_of(blocks, slots)
