@@ -969,11 +969,11 @@ static int enqueue_subchain(prism_ctx* c, const ChainWs& ws, const ChainPlan& pl
             if (!rc) rc = timer_mark(c, tm, 1, s);
             if (rc) return rc;
         } else if (!last) { /* one launch: attention + the FFN */
-            int rc = enqueue_attn(c, k, src, dst, H, W, nf, s, nullptr, first, true, plan.split);
+            int rc = enqueue_attn(c, k, src, dst, H, W, nf, s, nullptr, first, true, plan.par);
             if (!rc) rc = timer_mark(c, tm, 0, s);
             if (rc) return rc;
         } else {
-            int rc = enqueue_attn(c, k, src, attn, H, W, nf, s, nullptr, first, false, plan.split);
+            int rc = enqueue_attn(c, k, src, attn, H, W, nf, s, nullptr, first, false, plan.par);
             if (!rc) rc = timer_mark(c, tm, 0, s);
             if (!rc) rc = enqueue_experts(c, k, attn, dst, nullptr, nullptr, n, s, 1, last);
             if (!rc) rc = timer_mark(c, tm, 1, s);

@@ -30,6 +30,7 @@ static_assert(CHAIN_SPLIT >= 1 && CHAIN_SPLIT <= 4, "sub-chain streams");
 struct ChainPlan {
     int split;       /* sub-chains */
     bool one_launch; /* a dense chain: every block in one launch */
+    int par;         /* the sub-chains whose attention launches' windows count together (attn_w8) */
 };
 
 /* Sub-chains. A routed block's two launches leave CUs idle in
@@ -50,12 +51,32 @@ struct ChainPlan {
  * 267 -> 229 and 339 -> 300 us; of 540 windows, whose second round is nearly
  * empty for all 12 blocks, 393 and 430; of 1,080, 699 and 739. At d128, whose
  * windows are short, always: 4 blocks of 135, 540, 1,080 and 2,160 windows
- * 38 -> 31, 72 -> 57, 104 -> 98 and 182 -> 172 us. */
+ * 38 -> 31, 72 -> 57, 104 -> 98 and 182 -> 172 us.
+ *
+ * 257 windows and more in one launch are 4-wave workgroups, and the launch
+ * takes as long as the two that share a CU through all blocks, 272-280 us for
+ * 12 blocks, be it a few CUs or all. Two sub-chains of 8-wave launches, a
+ * block each, share the work out again at every block, and their time goes by
+ * the amount of it, a window whose lower half is padding (attn.hpp's HALF)
+ * counting two thirds. One launch against two sub-chains, by windows (of these
+ * half): 264 (88) 274 and 228 us, 264 (0) 274 and 263, 300 (100) 272 and 256,
+ * 300 (150) 272 and 243, 315 (63) 272 and 263, 336 (0) 282 and 282, 350 (70)
+ * 277 and 278, 360 (0) 281 and 301, 385 (77) 283 and 299, 420 (210) 280 and
+ * 285. So sub-chains up to 4/3 window per CU, but one launch where the
+ * windows past the 256th are all half ones, the last row of the last frame:
+ * 258 (129) 217 and 225, 270 (30) 222 and 236. */
 inline ChainPlan chain_plan(const prism_model_desc& d, int batch) {
-    const int64_t windows = (int64_t)((d.spatial_w + 7) / 8) * ((d.spatial_h + 7) / 8) * batch;
-    if (d.n_experts > 1) return {windows > CHAIN_SPLIT_ROUTED ? std::min(CHAIN_SPLIT, batch) : 1, false};
-    if (d.dim == 128 || windows <= 2 * CU_COUNT) return {1, true};
-    return {windows > CHAIN_SPLIT_DENSE ? std::min(CHAIN_SPLIT, batch) : 1, false};
+    const int64_t wx = (d.spatial_w + 7) / 8, windows = wx * ((d.spatial_h + 7) / 8) * batch;
+    if (d.n_experts > 1) return {windows > CHAIN_SPLIT_ROUTED ? std::min(CHAIN_SPLIT, batch) : 1, false, 1};
+    if (d.dim == 128) return {1, true, 1};
+    if (windows > CHAIN_SPLIT_DENSE) {
+        const int split = std::min(CHAIN_SPLIT, batch);
+        return {split, false, split};
+    }
+    const int64_t half = d.spatial_h % 8 >= 1 && d.spatial_h % 8 <= 4 ? wx : 0; /* a frame */
+    if (windows > CU_COUNT + half && 3 * windows - half * batch <= 4 * CU_COUNT && batch > 1)
+        return {CHAIN_SPLIT, false, 1};
+    return {1, true, 1};
 }
 
 /* Attention: 8 waves (a workgroup per CU at d256)? Windows that fit the CUs as
@@ -67,8 +88,9 @@ inline ChainPlan chain_plan(const prism_model_desc& d, int batch) {
  * takes 16.8 us on 8. Two d128 ones share a CU (270 windows 13.0 us either
  * way, 405 16.3 and 16.0). par: attention launches of about this size that run
  * at the same time (a dense chain's sub-chains; a routed one's run beside the
- * other's experts); their windows count together (two dense launches of 256 at
- * once: 162 us a four-block chain on 8 waves, 134 on 4). */
+ * other's experts) and whose windows count together (two dense launches of 256
+ * at once: 162 us a four-block chain on 8 waves, 134 on 4; two of at most 4/3
+ * window per CU together stay on 8, see chain_plan). */
 inline bool attn_w8(int dim, int64_t windows, int par) {
     return windows * par < (dim == 256 ? CU_COUNT + 1 : 2 * CU_COUNT);
 }

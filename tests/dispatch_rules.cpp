@@ -18,6 +18,11 @@ int chain(int dim, int experts, int h, int w, int batch) {
     const ChainPlan p = chain_plan(desc(dim, experts, h, w), batch);
     return p.one_launch ? -p.split : p.split;
 }
+/* of the first sub-chain's launches */
+int chain_attention_waves(int dim, int experts, int h, int w, int batch) {
+    const ChainPlan p = chain_plan(desc(dim, experts, h, w), batch);
+    return attn_w8(dim, (long long)((w + 7) / 8) * ((h + 7) / 8) * (batch / p.split), p.par) ? 8 : 4;
+}
 int attention_waves(int dim, long long windows, int par) { return attn_w8(dim, windows, par) ? 8 : 4; }
 long long projection_grid(int dim, long long tiles) { return project_grid(dim, tiles); }
 int enc2_slots(long long blocks) { return codec_enc2_slots(blocks); }

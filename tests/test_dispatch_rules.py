@@ -30,6 +30,13 @@ def rules(tmp_path_factory):
     (128, 1, 68, 120, 1, ONE), (128, 1, 68, 120, 16, ONE),  # d128: always together
     (256, 1, 64, 64, 4, ONE),                              # 256 windows
     (256, 1, 64, 64, 8, ONE), (256, 1, 64, 64, 9, 2),      # 512 | 576
+    # 257 to 341 windows' worth of work, a half-padded one counting 2/3: sub-chains
+    (256, 1, 24, 32, 22, 2), (256, 1, 24, 32, 28, 2), (256, 1, 24, 32, 29, ONE),  # 264, 336 | 348
+    (256, 1, 17, 25, 22, 2), (256, 1, 17, 25, 31, 2), (256, 1, 17, 25, 33, ONE),  # 372 (124 half) | 396 (132)
+    (256, 1, 25, 33, 16, 2), (256, 1, 80, 80, 3, 2), (256, 1, 96, 88, 2, 2),      # 320 (80), 300, 264
+    (256, 1, 21, 28, 28, 2), (256, 1, 20, 28, 33, ONE),    # 5 rows: no half ones, 336 | 4 rows: 396 (132)
+    (256, 1, 68, 120, 2, ONE), (256, 1, 9, 24, 43, ONE),   # only half windows past the 256th
+    (256, 1, 136, 128, 1, ONE),                            # 272 windows of one frame
     (256, 1, 135, 240, 2, 2),
 ])
 def test_chain_plan(rules, dim, experts, h, w, batch, plan):
@@ -38,6 +45,7 @@ def test_chain_plan(rules, dim, experts, h, w, batch, plan):
 
 def test_attention_waves(rules):
     assert [rules.attention_waves(256, n, 1) for n in (1, 256, 257)] == [8, 8, 4]
+    assert [rules.chain_attention_waves(256, 1, 24, 32, b) for b in (21, 22, 28, 29, 43)] == [8, 8, 8, 4, 4]
     assert [rules.attention_waves(128, n, 1) for n in (511, 512)] == [8, 4]
 
 
