@@ -589,12 +589,23 @@ extern "C" __global__ void __launch_bounds__(256, 2) prism_expert_d128_bm64(Expe
     __shared__ ExpertLds<128, 64> lds;
     expert_body<128, 64, 4>(a, lds);
 }
+/* The 8-wave d256 kernel asks for so much LDS that no attention window's 75 KB
+ * fits beside it, although a tile needs 70 KB. Measured, not derived (by their
+ * registers the two do not fit a CU either): where two sub-chains run, their
+ * launches follow one another better that way. 5 frames of 68x120, 64 experts
+ * 943 -> 874 us, 16 experts 882 -> 813; 4 frames, 16 experts 731 -> 700, 32
+ * experts 1,007 -> 987 (140 KB: the same); a launch alone takes as long as
+ * with 70 KB. */
+static constexpr int EXPERT_W8_LDS = 90 * 1024;
 extern "C" __global__ void __launch_bounds__(512, 1) prism_expert_d256_bm64_w8(ExpertArgs a) {
-    __shared__ ExpertLds<256, 64> lds;
+    __shared__ union {
+        ExpertLds<256, 64> tile;
+        unsigned char whole[EXPERT_W8_LDS];
+    } lds;
     if (a.wnt) /* uniform */
-        expert_body<256, 64, 8, true>(a, lds);
+        expert_body<256, 64, 8, true>(a, lds.tile);
     else
-        expert_body<256, 64, 8>(a, lds);
+        expert_body<256, 64, 8>(a, lds.tile);
 }
 extern "C" __global__ void __launch_bounds__(512, 1) prism_expert_d128_bm64_w8(ExpertArgs a) {
     __shared__ ExpertLds<128, 64> lds;

@@ -133,3 +133,27 @@ def test_expert_stage_at_the_edge_of_one_round(hip, engine, device_arena, name, 
         hip.sync()
         ys.append(hip.download(np.empty(T * d, np.uint16), feats.ptr + x.nbytes))
     assert (ys[0] == ys[1]).all()
+
+
+@pytest.mark.gpu
+def test_no_lds_beside_an_8_wave_expert_tile_for_an_attention_window(hip):
+    """160 KB a CU; sub-chains run slower where there is."""
+    import ctypes as C
+    import os
+
+    rt, mod, fn = C.CDLL("libamdhip64.so"), C.c_void_p(), C.c_void_p()
+    path = os.path.join(os.path.dirname(os.path.abspath(P.__file__)), "prism_kernels.hsaco")
+    assert rt.hipModuleLoad(C.byref(mod), path.encode()) == 0
+
+    def lds(kernel):
+        v = C.c_int()
+        assert rt.hipModuleGetFunction(C.byref(fn), mod, kernel.encode()) == 0
+        assert rt.hipFuncGetAttribute(C.byref(v), 1, fn) == 0  # HIP_FUNC_ATTRIBUTE_SHARED_SIZE_BYTES
+        return v.value
+
+    try:
+        least = min(lds(f"prism_attn_d256{w}_r{r}") for w in ("", "_w8") for r in (1, 2, 3, 4))
+        assert 64 * 1024 < least < 80 * 1024
+        assert lds("prism_expert_d256_bm64_w8") + least > 160 * 1024
+    finally:
+        assert rt.hipModuleUnload(mod) == 0
