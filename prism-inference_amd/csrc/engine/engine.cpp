@@ -486,14 +486,13 @@ struct RouteOut {
     RouteTake take;     /* stage calls: where the totals go */
 };
 
-/* par: attention launches of about this size that run at the same time (a
- * dense chain's sub-chains; a routed one's run beside the other's experts).
+/* plan: the chain's (NULL: a stage call).
  * ffn: a dense block's FFN runs in the same launch (the window's rows never
  * leave the CU between the two), and `out` receives the block's output.
  * blocks > 1: that many dense blocks from k on in one launch */
 int enqueue_attn(prism_ctx* c, const DevBlock& k, const uint16_t* in, uint16_t* out, int H, int W, int batch,
-                 hipStream_t s, const RouteOut* route = nullptr, bool up = false, bool ffn = false, int par = 1,
-                 int blocks = 1) {
+                 hipStream_t s, const RouteOut* route = nullptr, const ChainPlan* plan = nullptr, bool up = false,
+                 bool ffn = false, int blocks = 1) {
     const int D = c->desc.dim;
     if (ffn && (route || c->desc.n_experts != 1))
         return fail(c, PRISM_ERR_INVALID, "the fused FFN is for dense blocks");
@@ -538,7 +537,7 @@ int enqueue_attn(prism_ctx* c, const DevBlock& k, const uint16_t* in, uint16_t* 
     }
     const int64_t grid = (int64_t)a.windows_per_frame * batch;
     if (grid <= 0 || grid > 0x7fffffff) return fail(c, PRISM_ERR_INVALID, "attention grid %lld out of range", (long long)grid);
-    const int w8 = attn_w8(D, grid, par) ? 1 : 0;
+    const int w8 = (plan ? chain_attn_w8(c->desc, *plan, grid) : attn_w8(D, grid)) ? 1 : 0;
     if (blocks > 1) {
         const DevBlock* const kb = &k;
         a.n_blocks = blocks;
@@ -588,7 +587,7 @@ int enqueue_router(prism_ctx* c, const DevBlock& k, const uint16_t* in, int32_t*
 
 int enqueue_experts(prism_ctx* c, const DevBlock& k, const uint16_t* in, uint16_t* out, const int32_t* counts,
                     const int32_t* perm, int64_t n, hipStream_t s, int32_t count_stride = 1, bool dn = false,
-                    bool stage = false, bool wnt = false) {
+                    const ChainPlan* plan = nullptr, bool wnt = false) {
     const int D = c->desc.dim, N = counts ? c->desc.n_experts : 1;
     ExpertArgs a{};
     if (dn) { /* the adapted chain's last block: 128-channel output rows */
@@ -612,10 +611,10 @@ int enqueue_experts(prism_ctx* c, const DevBlock& k, const uint16_t* in, uint16_
      * a multiple of 8 (the kernels' XCD-major tile order) */
     auto tiles_of = [&](int64_t bm) { return ((n + bm - 1) / bm + (counts ? N : 0) + 7) / 8 * 8; };
     if (D == 256 && !dn && tiles_of(128) >= EXPERT_WIDE_MIN_TILES)
-        return stage ? launch(c, c->f_expert_wide96, (unsigned)tiles_of(96), a, s, 256u)
-                     : launch(c, c->f_expert_wide, (unsigned)tiles_of(128), a, s, 256u);
+        return plan ? launch(c, c->f_expert_wide, (unsigned)tiles_of(128), a, s, 256u)
+                    : launch(c, c->f_expert_wide96, (unsigned)tiles_of(96), a, s, 256u);
     const int64_t tiles = tiles_of(64);
-    const int w8 = expert_w8(D, tiles, n, counts ? N : 0, stage) ? 1 : 0;
+    const int w8 = expert_w8(D, tiles, n, counts ? N : 0, plan) ? 1 : 0;
     return launch(c, c->f_expert[dim_index(D)][w8], (unsigned)tiles, a, s, w8 ? 512u : 256u);
 }
 
@@ -794,7 +793,7 @@ extern "C" int prism_experts(prism_ctx* c, const prism_expert_push* p, void* fea
         return fail(c, PRISM_ERR_INVALID, "feature offsets must be multiples of 8 elements");
     HIP_TRY(c, hipSetDevice(c->device));
     return enqueue_experts(c, *k, f + p->input_offset, f + p->output_offset, dense ? nullptr : aux + p->count_offset,
-                           dense ? nullptr : aux + p->perm_offset, n, (hipStream_t)stream, 1, false, true);
+                           dense ? nullptr : aux + p->perm_offset, n, (hipStream_t)stream, 1);
 }
 
 static int project_stage(prism_ctx* c, bool up, const prism_project_push* p, void* features, int32_t batch,
@@ -945,7 +944,7 @@ static int enqueue_subchain(prism_ctx* c, const ChainWs& ws, const ChainPlan& pl
         b0 = adapted ? NB - 1 : NB;
         if (b0 > 1) {
             uint16_t* dst = b0 == NB ? out : scratch;
-            int rc = enqueue_attn(c, c->blocks[0], src, dst, H, W, nf, s, nullptr, adapted, true, 1, b0);
+            int rc = enqueue_attn(c, c->blocks[0], src, dst, H, W, nf, s, nullptr, &plan, adapted, true, b0);
             if (!rc) rc = timer_mark(c, tm, 0, s);
             if (rc) return rc;
             src = dst;
@@ -961,21 +960,21 @@ static int enqueue_subchain(prism_ctx* c, const ChainWs& ws, const ChainPlan& pl
             int32_t* counts = counts0 + (size_t)b * row;
             const RouteOut ro{ws.assign + (size_t)b * n_all + t0, counts, perm, CHAIN_COUNT_STRIDE,
                               NB > 1 ? counts0 + (size_t)((b + 1) % NB) * row : nullptr, RouteTake{}};
-            int rc = enqueue_attn(c, k, src, attn, H, W, nf, s, &ro, first);
+            int rc = enqueue_attn(c, k, src, attn, H, W, nf, s, &ro, &plan, first);
             if (!rc) rc = timer_mark(c, tm, 0, s);
             if (!rc)
-                rc = enqueue_experts(c, k, attn, dst, counts, perm, n, s, CHAIN_COUNT_STRIDE, last, false,
+                rc = enqueue_experts(c, k, attn, dst, counts, perm, n, s, CHAIN_COUNT_STRIDE, last, &plan,
                                      b < c->wnt_blocks);
             if (!rc) rc = timer_mark(c, tm, 1, s);
             if (rc) return rc;
         } else if (!last) { /* one launch: attention + the FFN */
-            int rc = enqueue_attn(c, k, src, dst, H, W, nf, s, nullptr, first, true, plan.par);
+            int rc = enqueue_attn(c, k, src, dst, H, W, nf, s, nullptr, &plan, first, true);
             if (!rc) rc = timer_mark(c, tm, 0, s);
             if (rc) return rc;
         } else {
-            int rc = enqueue_attn(c, k, src, attn, H, W, nf, s, nullptr, first, false, plan.par);
+            int rc = enqueue_attn(c, k, src, attn, H, W, nf, s, nullptr, &plan, first);
             if (!rc) rc = timer_mark(c, tm, 0, s);
-            if (!rc) rc = enqueue_experts(c, k, attn, dst, nullptr, nullptr, n, s, 1, last);
+            if (!rc) rc = enqueue_experts(c, k, attn, dst, nullptr, nullptr, n, s, 1, last, &plan);
             if (!rc) rc = timer_mark(c, tm, 1, s);
             if (rc) return rc;
         }

@@ -30,7 +30,8 @@ static_assert(CHAIN_SPLIT >= 1 && CHAIN_SPLIT <= 4, "sub-chain streams");
 struct ChainPlan {
     int split;       /* sub-chains */
     bool one_launch; /* a dense chain: every block in one launch */
-    int par;         /* the sub-chains whose attention launches' windows count together (attn_w8) */
+    bool pair8;      /* both sub-chains' launches on 8 waves */
+    int64_t windows; /* of the batch */
 };
 
 /* Sub-chains. A routed block's two launches leave CUs idle in
@@ -64,19 +65,37 @@ struct ChainPlan {
  * 277 and 278, 360 (0) 281 and 301, 385 (77) 283 and 299, 420 (210) 280 and
  * 285. So sub-chains up to 4/3 window per CU, but one launch where the
  * windows past the 256th are all half ones, the last row of the last frame:
- * 258 (129) 217 and 225, 270 (30) 222 and 236. */
+ * 258 (129) 217 and 225, 270 (30) 222 and 236.
+ *
+ * The waves of two sub-chains (chain_attn_w8). The launches of a dense chain's
+ * are on 8 together, up to 4/3 window per CU, or on 4 (two of 256 at once: 162
+ * us a four-block chain on 8 waves, 134 on 4). A routed sub-chain's go by its
+ * own windows, except that with more than 32 experts, 513 to CHAIN_PAIR8_MAX
+ * windows in about equal halves and expert launches of more than
+ * CHAIN_PAIR8_TILES tiles attention and experts both stay on 8 waves. 64 experts, both on 8, attention on 4,
+ * both on 4: 4 frames of 68x120 (2 x 270 windows, 319 tiles) 759, 779 and 804
+ * us, of 66x118 (307 tiles) 740, 750 and 782, of 72x120 782, 791 and 831; 22
+ * of 24x64 (2 x 264) 771, 780 and 797; 23 804, 819 and 830; but 24 (2 x 288)
+ * 819, 827 and 806, 4 of 65x121 (2 x 288, 310 tiles) 774, 759 and 806, 16 of
+ * 33x51 (2 x 280, 275 tiles) 795 and 750. With 32 experts (4 of 72x120: 1,034,
+ * 983 and 1,004) or 16 (732, 701 and 714) the windows alone decide. */
+constexpr int CHAIN_PAIR8_MAX = CU_COUNT * 11 / 5, CHAIN_PAIR8_TILES = CU_COUNT * 7 / 6;
 inline ChainPlan chain_plan(const prism_model_desc& d, int batch) {
-    const int64_t wx = (d.spatial_w + 7) / 8, windows = wx * ((d.spatial_h + 7) / 8) * batch;
-    if (d.n_experts > 1) return {windows > CHAIN_SPLIT_ROUTED ? std::min(CHAIN_SPLIT, batch) : 1, false, 1};
-    if (d.dim == 128) return {1, true, 1};
-    if (windows > CHAIN_SPLIT_DENSE) {
-        const int split = std::min(CHAIN_SPLIT, batch);
-        return {split, false, split};
+    const int64_t wx = (d.spatial_w + 7) / 8, frame = wx * ((d.spatial_h + 7) / 8), windows = frame * batch;
+    if (d.n_experts > 1) {
+        const int split = windows > CHAIN_SPLIT_ROUTED ? std::min(CHAIN_SPLIT, batch) : 1;
+        const int64_t tokens = (int64_t)d.spatial_w * d.spatial_h * batch;
+        const bool pair8 = split > 1 && d.dim == 256 && d.n_experts > 32 && windows > 2 * CU_COUNT &&
+                           windows <= CHAIN_PAIR8_MAX && (batch + 1) / 2 * frame <= CU_COUNT * 9 / 8 &&
+                           tokens / 128 + d.n_experts > CHAIN_PAIR8_TILES;
+        return {split, false, pair8, windows};
     }
+    if (d.dim == 128) return {1, true, false, windows};
+    if (windows > CHAIN_SPLIT_DENSE) return {std::min(CHAIN_SPLIT, batch), false, false, windows};
     const int64_t half = d.spatial_h % 8 >= 1 && d.spatial_h % 8 <= 4 ? wx : 0; /* a frame */
     if (windows > CU_COUNT + half && 3 * windows - half * batch <= 4 * CU_COUNT && batch > 1)
-        return {CHAIN_SPLIT, false, 1};
-    return {1, true, 1};
+        return {CHAIN_SPLIT, false, true, windows};
+    return {1, true, false, windows};
 }
 
 /* Attention: 8 waves (a workgroup per CU at d256)? Windows that fit the CUs as
@@ -86,17 +105,19 @@ inline ChainPlan chain_plan(const prism_model_desc& d, int batch) {
  * starts a second round: routed launches of 270, 405 and 510 windows take
  * 28.6, 32.6 and 35 us on 8 waves, 23.6, 27.5 and 30.7 on 4, and one of 135
  * takes 16.8 us on 8. Two d128 ones share a CU (270 windows 13.0 us either
- * way, 405 16.3 and 16.0). par: attention launches of about this size that run
- * at the same time (a dense chain's sub-chains; a routed one's run beside the
- * other's experts) and whose windows count together (two dense launches of 256
- * at once: 162 us a four-block chain on 8 waves, 134 on 4; two of at most 4/3
- * window per CU together stay on 8, see chain_plan). */
-inline bool attn_w8(int dim, int64_t windows, int par) {
-    return windows * par < (dim == 256 ? CU_COUNT + 1 : 2 * CU_COUNT);
+ * way, 405 16.3 and 16.0). */
+inline bool attn_w8(int dim, int64_t windows) { return windows <= (dim == 256 ? CU_COUNT : 2 * CU_COUNT - 1); }
+
+/* The same for a chain's launch of `windows` (chain_plan). */
+inline bool chain_attn_w8(const prism_model_desc& d, const ChainPlan& p, int64_t windows) {
+    if (p.pair8) return true;
+    if (d.dim == 256 && p.split > 1 && d.n_experts == 1) return false;
+    return attn_w8(d.dim, windows);
 }
 
 /* Experts, 64-token tiles: 8 waves? tiles: the launch's grid, n / 64 and a
- * partial tile per expert; n: its tokens; partial: the experts (0 if dense).
+ * partial tile per expert; n: its tokens; partial: the experts (0 if dense);
+ * p: the chain's plan, NULL for a stage call.
  * At most one tile per CU: 8 waves per tile halve each wave's weight
  * stream; otherwise 4 waves x 2 tiles per CU. Alone on the GPU what counts
  * is the tiles that hold tokens, about half a tile per expert more than
@@ -107,9 +128,10 @@ inline bool attn_w8(int dim, int64_t windows, int par) {
  * with launches of 280 tiles 696 us on 8 waves, 770 on 4; of 296, 745 and
  * 789; of 320, 816 and 832 (or 807 and 789); of 352, 891 and 855. d128
  * tiles leave room for two 8-wave workgroups per CU. */
-inline bool expert_w8(int dim, int64_t tiles, int64_t n, int partial, bool stage) {
+inline bool expert_w8(int dim, int64_t tiles, int64_t n, int partial, const ChainPlan* p) {
     if (dim != 256) return tiles < 2 * CU_COUNT;
-    return stage ? (n + 63) / 64 + partial / 2 <= CU_COUNT : tiles <= CU_COUNT * 5 / 4;
+    if (p && p->pair8) return true;
+    return !p ? (n + 63) / 64 + partial / 2 <= CU_COUNT : tiles <= CU_COUNT * 5 / 4;
 }
 
 /* ---- projection stages */

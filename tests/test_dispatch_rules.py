@@ -17,7 +17,7 @@ def rules(tmp_path_factory):
                     "-I", os.path.join(HERE, "..", "include"), os.path.join(HERE, "dispatch_rules.cpp"), "-o", so],
                    check=True, timeout=120)
     lib = C.CDLL(so)
-    lib.attention_waves.argtypes = [C.c_int, C.c_longlong, C.c_int]
+    lib.attention_waves.argtypes = [C.c_int, C.c_longlong]
     lib.projection_grid.argtypes, lib.projection_grid.restype = [C.c_int, C.c_longlong], C.c_longlong
     lib.enc2_slots.argtypes = [C.c_longlong]
     lib.grid_of.argtypes, lib.grid_of.restype = [C.c_longlong, C.c_int], C.c_uint
@@ -44,9 +44,25 @@ def test_chain_plan(rules, dim, experts, h, w, batch, plan):
 
 
 def test_attention_waves(rules):
-    assert [rules.attention_waves(256, n, 1) for n in (1, 256, 257)] == [8, 8, 4]
+    assert [rules.attention_waves(256, n) for n in (1, 256, 257)] == [8, 8, 4]
     assert [rules.chain_attention_waves(256, 1, 24, 32, b) for b in (21, 22, 28, 29, 43)] == [8, 8, 8, 4, 4]
-    assert [rules.attention_waves(128, n, 1) for n in (511, 512)] == [8, 4]
+    assert [rules.attention_waves(128, n) for n in (511, 512)] == [8, 4]
+
+
+@pytest.mark.parametrize("experts,h,w,batch,attention,expert", [
+    (64, 64, 64, 8, 8, 8),        # 512 windows: 256 a sub-chain, 320 tiles
+    (64, 68, 120, 4, 8, 8),       # 540: both on 8 waves
+    (64, 72, 120, 4, 8, 8),       # ... also at 334 tiles
+    (64, 66, 118, 4, 8, 8),       # 307 tiles
+    (64, 33, 51, 16, 4, 8),       # 275 tiles
+    (64, 24, 64, 24, 4, 4),       # 576 windows
+    (32, 68, 120, 4, 4, 8), (16, 68, 120, 4, 4, 8), (16, 72, 120, 5, 4, 4),
+    (64, 24, 64, 23, 8, 8), (64, 96, 120, 3, 4, 4),  # 264 and 288 | 180 and 360: unequal halves
+    (64, 68, 120, 16, 4, 4),
+])
+def test_waves_of_routed_sub_chains(rules, experts, h, w, batch, attention, expert):
+    assert rules.chain_attention_waves(256, experts, h, w, batch) == attention
+    assert rules.chain_expert_waves(256, experts, h, w, batch) == expert
 
 
 @pytest.mark.parametrize("blocks,grid", [(256, 256), (257, 129), (510, 255), (1024, 256), (1025, 342), (2040, 510)])
