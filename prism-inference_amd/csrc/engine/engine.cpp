@@ -587,7 +587,7 @@ int enqueue_router(prism_ctx* c, const DevBlock& k, const uint16_t* in, int32_t*
 
 int enqueue_experts(prism_ctx* c, const DevBlock& k, const uint16_t* in, uint16_t* out, const int32_t* counts,
                     const int32_t* perm, int64_t n, hipStream_t s, int32_t count_stride = 1, bool dn = false,
-                    const ChainPlan* plan = nullptr, bool wnt = false) {
+                    const ChainPlan* plan = nullptr, bool leading = false) {
     const int D = c->desc.dim, N = counts ? c->desc.n_experts : 1;
     ExpertArgs a{};
     if (dn) { /* the adapted chain's last block: 128-channel output rows */
@@ -606,7 +606,6 @@ int enqueue_experts(prism_ctx* c, const DevBlock& k, const uint16_t* in, uint16_
     a.n_experts = N;
     a.cap = (int32_t)n;
     a.count_stride = count_stride;
-    a.wnt = wnt ? 1 : 0;
     /* tiles: the worst case of ceil(n / bm) + one partial tile per expert,
      * a multiple of 8 (the kernels' XCD-major tile order) */
     auto tiles_of = [&](int64_t bm) { return ((n + bm - 1) / bm + (counts ? N : 0) + 7) / 8 * 8; };
@@ -615,6 +614,7 @@ int enqueue_experts(prism_ctx* c, const DevBlock& k, const uint16_t* in, uint16_
                     : launch(c, c->f_expert_wide96, (unsigned)tiles_of(96), a, s, 256u);
     const int64_t tiles = tiles_of(64);
     const int w8 = expert_w8(D, tiles, n, counts ? N : 0, plan) ? 1 : 0;
+    a.wnt = plan && expert_wnt(leading, w8, *plan) ? 1 : 0;
     return launch(c, c->f_expert[dim_index(D)][w8], (unsigned)tiles, a, s, w8 ? 512u : 256u);
 }
 

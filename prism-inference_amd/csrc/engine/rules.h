@@ -134,6 +134,14 @@ inline bool expert_w8(int dim, int64_t tiles, int64_t n, int partial, const Chai
     return !p ? (n + 63) / 64 + partial / 2 <= CU_COUNT : tiles <= CU_COUNT * 5 / 4;
 }
 
+/* The leading blocks' expert weights are read past the memory-side cache
+ * (ctx.h's WEIGHT_CACHE_KEEP) by 8-wave launches, and by 4-wave ones of a chain
+ * without sub-chains (64 experts, one frame of 135x240: 842 -> 815 us). Two
+ * sub-chains read a block's weights one after the other, and what the first
+ * left in that cache is worth more: 8 frames of 68x120 1,277 -> 1,266 us on
+ * plain loads, 10 frames 1,543 -> 1,527. */
+inline bool expert_wnt(bool leading, bool w8, const ChainPlan& p) { return leading && (w8 || p.split == 1); }
+
 /* ---- projection stages */
 
 /* Workgroups of a projection stage launch (persistent, 64-token tiles in a

@@ -30,6 +30,11 @@ int chain_expert_waves(int dim, int experts, int h, int w, int batch) {
     const long long n = (long long)h * w * last_frames(p, batch), tiles = ((n + 63) / 64 + partial + 7) / 8 * 8;
     return expert_w8(dim, tiles, n, partial, &p) ? 8 : 4;
 }
+/* the leading blocks' expert weights past the memory-side cache? */
+int chain_expert_streams(int dim, int experts, int h, int w, int batch) {
+    return expert_wnt(true, chain_expert_waves(dim, experts, h, w, batch) == 8,
+                      chain_plan(desc(dim, experts, h, w), batch));
+}
 int attention_waves(int dim, long long windows) { return attn_w8(dim, windows) ? 8 : 4; }
 long long projection_grid(int dim, long long tiles) { return project_grid(dim, tiles); }
 int enc2_slots(long long blocks) { return codec_enc2_slots(blocks); }

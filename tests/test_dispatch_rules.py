@@ -65,6 +65,14 @@ def test_waves_of_routed_sub_chains(rules, experts, h, w, batch, attention, expe
     assert rules.chain_expert_waves(256, experts, h, w, batch) == expert
 
 
+@pytest.mark.parametrize("h,w,batch,streams", [
+    (68, 120, 1, True), (68, 120, 2, True), (135, 240, 1, True),  # 8 waves | 4 waves, one chain
+    (68, 120, 8, False), (68, 120, 10, False),                    # 4 waves beside another sub-chain
+])
+def test_leading_blocks_weights_past_the_cache(rules, h, w, batch, streams):
+    assert bool(rules.chain_expert_streams(256, 64, h, w, batch)) == streams
+
+
 @pytest.mark.parametrize("blocks,grid", [(256, 256), (257, 129), (510, 255), (1024, 256), (1025, 342), (2040, 510)])
 def test_enc2_keeps_to_one_workgroup_per_cu(rules, blocks, grid):
     """Two per CU pull the clock down for the chain that follows."""
