@@ -89,6 +89,7 @@ struct prism_ctx {
     hipFunction_t f_expert_wide96 = nullptr; /* d256, 96-token tiles (large stage calls) */
     hipFunction_t f_zero = nullptr;
     hipFunction_t f_proj[2][2] = {};    /* [dim][up, down] */
+    hipFunction_t f_proj_down_w8 = nullptr; /* d256 down, 8 waves */
     hipFunction_t f_codec[7] = {};     /* enc0..enc3, dec3, dec2, dec1_out */
     hipFunction_t f_codec21 = nullptr; /* dec2 + dec1_out in one launch (the decoder's last two stages) */
     hipFunction_t f_enc01 = nullptr;   /* enc0 + enc1 in one launch (the encoder's first two stages) */

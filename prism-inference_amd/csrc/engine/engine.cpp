@@ -104,8 +104,9 @@ extern "C" int prism_create(prism_ctx** out, int32_t device, const char* code_ob
         {&c->f_expert[0][1], "prism_expert_d128_bm64_w8"}, {&c->f_expert[1][1], "prism_expert_d256_bm64_w8"},
         {&c->f_expert_wide, "prism_expert_d256_bm128"}, {&c->f_expert_wide96, "prism_expert_d256_bm96"},
         {&c->f_zero, "prism_zero_i32"},
-        {&c->f_proj[0][0], "prism_project_up_d128"},   {&c->f_proj[0][1], "prism_project_down_d128"},
-        {&c->f_proj[1][0], "prism_project_up_d256"},   {&c->f_proj[1][1], "prism_project_down_d256"},
+        {&c->f_proj[0][0], "prism_project_up_d128"},      {&c->f_proj[0][1], "prism_project_down_d128"},
+        {&c->f_proj[1][0], "prism_project_up_d256_w8"},   {&c->f_proj[1][1], "prism_project_down_d256"},
+        {&c->f_proj_down_w8, "prism_project_down_d256_w8"},
         {&c->f_codec[0], "prism_codec_enc0"}, {&c->f_codec[1], "prism_codec_enc1"},
         {&c->f_codec[2], "prism_codec_enc2"}, {&c->f_codec[3], "prism_codec_enc3"},
         {&c->f_codec[4], "prism_codec_dec3"}, {&c->f_codec[5], "prism_codec_dec2"},
@@ -630,7 +631,9 @@ int enqueue_project(prism_ctx* c, bool up, const uint16_t* in, uint16_t* out, in
     if (tiles <= 0 || tiles > 0x7fffffff) return fail(c, PRISM_ERR_INVALID, "projection tiles %lld out of range", (long long)tiles);
     /* persistent workgroups looping over 64-token tiles */
     const int D = c->desc.dim;
-    return launch(c, c->f_proj[dim_index(D)][up ? 0 : 1], (unsigned)project_grid(D, tiles), a, s, D == 256 ? 512u : 256u);
+    const bool w8 = project_w8(D, up, tiles);
+    return launch(c, w8 && !up ? c->f_proj_down_w8 : c->f_proj[dim_index(D)][up ? 0 : 1], (unsigned)project_grid(D, tiles), a,
+                  s, w8 ? 512u : 256u);
 }
 
 /* which: 0 = attention (qkv_w), 1 = router (router_w), 2 = experts (exp_w1) */

@@ -145,14 +145,19 @@ inline bool expert_wnt(bool leading, bool w8, const ChainPlan& p) { return leadi
 /* ---- projection stages */
 
 /* Workgroups of a projection stage launch (persistent, 64-token tiles in a
- * loop, two per CU); at d256 up to PROJ_SINGLE_MAX tiles go one to a
- * workgroup. Both d256 launches, 765 tiles: 19.1 us on 512 workgroups, 18.3 on
- * 765; 2,040 tiles: 41.5 on 512, 43.7 on 768. */
-constexpr int PROJ_GRID_MAX = 512;
-constexpr int PROJ_SINGLE_MAX = 768;
+ * loop): PROJ_SLOTS, the two per CU that are resident; at d256 up to two
+ * rounds of them go a tile to a workgroup, which spreads a partial second
+ * round over the CUs. Both d256 launches, 700 tiles: 18.6 us on 512 workgroups,
+ * 18.0 on 700; 800: 21.9 and 20.4; 900: 22.5 and 20.9; 1,020: 23.5 and 22.2;
+ * but 1,500 32.3 and 34.6; 2,040 42.5 and 45.3. */
+constexpr int PROJ_SLOTS = 2 * CU_COUNT;
 inline int64_t project_grid(int dim, int64_t tiles) {
-    return dim == 256 && tiles <= PROJ_SINGLE_MAX ? tiles : std::min<int64_t>(tiles, PROJ_GRID_MAX);
+    return dim == 256 && tiles <= 2 * PROJ_SLOTS ? tiles : std::min<int64_t>(tiles, PROJ_SLOTS);
 }
+/* 8 waves: d256 (16 waves per CU instead of 8), but not the down-projection's
+ * persistent form, which they slow (2,040 tiles 21.3 us, 4 waves 20.6; up 19.0
+ * on either); at d128 4 waves are 4 % faster. */
+inline bool project_w8(int dim, bool up, int64_t tiles) { return dim == 256 && (up || tiles <= 2 * PROJ_SLOTS); }
 
 /* ---- codec */
 

@@ -9,7 +9,7 @@
  *   prism_chain_d{256,128}[_w8]                    every block of a dense chain in one launch
  *   prism_router_d{256,128}_n{1..4}                router + counting sort
  *   prism_expert_d{256,128}_bm64[_w8], _d256_bm{128,96}  grouped expert FFN
- *   prism_project_{up,down}_d{256,128}             projection adapters (128 <-> dim)
+ *   prism_project_{up,down}_d{256,128}[_w8]        projection adapters (128 <-> dim)
  *   prism_codec_enc{0,1}, prism_codec_dec2         conv encoder / fused decoder stages
  *   prism_codec_enc01, prism_codec_dec21_out       the same, fused in the frame (persistent)
  *   prism_codec_enc{2,3}, prism_codec_dec3         stages and frame alike (persistent)

@@ -12,9 +12,10 @@
  * tokens, accumulators starting at the bias. Persistent: workgroup b takes
  * tiles b, b + G, b + 2G, ... (G = the grid), holds its waves' weight
  * fragments in registers across them, and requests the next tile's rows
- * before the current tile's MFMAs. d256 on 8 waves (112 VGPRs, 16 waves per
- * CU instead of 8: both launches of 4 and 6 frames of 68x120 15.2 -> 13.9 and
- * 19.9 -> 18.3 us), d128 on 4 (8 measured 4 % slower).
+ * before the current tile's MFMAs. On 8 waves a wave holds half the weights
+ * (112 VGPRs, 16 waves per CU instead of 8: both d256 launches of 4 and 6
+ * frames of 68x120 15.2 -> 13.9 and 19.9 -> 18.3 us); which launches take
+ * them: project_w8 (engine/rules.h).
  */
 #pragma once
 #include "common.hpp"
@@ -119,11 +120,14 @@ __device__ __forceinline__ void project_body(const ProjArgs& a) {
 }
 
 /* up: encoder channels (128) -> model dim, ReLU; down: model dim -> 128 */
-extern "C" __global__ void __launch_bounds__(512, 4) prism_project_up_d256(ProjArgs a) {
+extern "C" __global__ void __launch_bounds__(512, 4) prism_project_up_d256_w8(ProjArgs a) {
     project_body<128, 256, true, 8>(a);
 }
-extern "C" __global__ void __launch_bounds__(512, 4) prism_project_down_d256(ProjArgs a) {
+extern "C" __global__ void __launch_bounds__(512, 4) prism_project_down_d256_w8(ProjArgs a) {
     project_body<256, 128, false, 8>(a);
+}
+extern "C" __global__ void __launch_bounds__(256, 2) prism_project_down_d256(ProjArgs a) {
+    project_body<256, 128, false, 4>(a);
 }
 extern "C" __global__ void __launch_bounds__(256, 2) prism_project_up_d128(ProjArgs a) {
     project_body<128, 128, true, 4>(a);

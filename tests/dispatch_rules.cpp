@@ -36,6 +36,7 @@ int chain_expert_streams(int dim, int experts, int h, int w, int batch) {
                       chain_plan(desc(dim, experts, h, w), batch));
 }
 int attention_waves(int dim, long long windows) { return attn_w8(dim, windows) ? 8 : 4; }
+int projection_waves(int dim, int up, long long tiles) { return project_w8(dim, up, tiles) ? 8 : 4; }
 long long projection_grid(int dim, long long tiles) { return project_grid(dim, tiles); }
 int enc2_slots(long long blocks) { return codec_enc2_slots(blocks); }
 unsigned grid_of(long long blocks, int slots) { return even_grid(blocks, slots); }

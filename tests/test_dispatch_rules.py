@@ -19,6 +19,7 @@ def rules(tmp_path_factory):
     lib = C.CDLL(so)
     lib.attention_waves.argtypes = [C.c_int, C.c_longlong]
     lib.projection_grid.argtypes, lib.projection_grid.restype = [C.c_int, C.c_longlong], C.c_longlong
+    lib.projection_waves.argtypes = [C.c_int, C.c_int, C.c_longlong]
     lib.enc2_slots.argtypes = [C.c_longlong]
     lib.grid_of.argtypes, lib.grid_of.restype = [C.c_longlong, C.c_int], C.c_uint
     return lib
@@ -71,6 +72,16 @@ def test_waves_of_routed_sub_chains(rules, experts, h, w, batch, attention, expe
 ])
 def test_leading_blocks_weights_past_the_cache(rules, h, w, batch, streams):
     assert bool(rules.chain_expert_streams(256, 64, h, w, batch)) == streams
+
+
+@pytest.mark.parametrize("dim,tiles,grid,up,down", [
+    (256, 1, 1, 8, 8), (256, 513, 513, 8, 8), (256, 900, 900, 8, 8), (256, 1024, 1024, 8, 8),
+    (256, 1025, 512, 8, 4), (256, 2040, 512, 8, 4),
+    (128, 512, 512, 4, 4), (128, 513, 512, 4, 4),
+])
+def test_projection_launches(rules, dim, tiles, grid, up, down):
+    assert rules.projection_grid(dim, tiles) == grid
+    assert (rules.projection_waves(dim, 1, tiles), rules.projection_waves(dim, 0, tiles)) == (up, down)
 
 
 @pytest.mark.parametrize("blocks,grid", [(256, 256), (257, 129), (510, 255), (1024, 256), (1025, 342), (2040, 510)])

@@ -190,3 +190,34 @@ def test_fused_adapters_equal_the_separate_calls(hip, engine, device_arena, name
         got = hip.download(np.empty(n * I, np.uint16), dy.ptr)
         assert (got == ref).all(), f"graph={graph}: {int((got != ref).sum())} values differ"
     assert np.isfinite(f16(ref)).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens", [64 * 513 - 5, 64 * 1024, 64 * 1024 + 1, 64 * 1100 - 63])
+def test_projection_rows_are_the_same_in_every_launch(hip, engine, device_arena, tokens):
+    """A tile a workgroup up to 1,024 tiles, persistent above (down on 4 waves):
+    the first and the last rows come out as in a call of their own."""
+    cfg, desc, blob, offs, ablob, a = setup(engine, "std256", 1, 8, 64)
+    D, I, m = cfg.dim, a.in_dim, 512
+    x = P.synth_normal(tokens * I, seed=12)
+    feats = device_arena(tokens * (2 * I + D) * 2)
+    push = [engine.project_push(True, m, 0, tokens * I), engine.project_push(False, m, tokens * I, tokens * (I + D))]
+    hip.upload(feats.ptr, x)
+
+    def run(n, first):
+        hip.memset(feats.ptr + tokens * I * 2, 0xFF, tokens * (I + D) * 2)
+        for up in (True, False):
+            p = push[not up]
+            p.n_tokens = n
+            p.input_offset = first * I if up else tokens * I
+            assert engine.project(up, p, feats.ptr, 1) == 0, engine.error()
+        hip.sync()
+        return (hip.download(np.empty((n, D), np.uint16), feats.ptr + tokens * I * 2),
+                hip.download(np.empty((n, I), np.uint16), feats.ptr + tokens * (I + D) * 2))
+
+    print(f"[proj] {tokens} tokens", flush=True)
+    whole = run(tokens, 0)
+    for first in (0, (tokens - m) // 64 * 64):
+        for got, ref in zip(whole, run(min(m, tokens - first), first)):
+            assert (got[first:first + len(ref)] == ref).all()
+    assert (whole[0] != 0xFFFF).all() and (whole[1] != 0xFFFF).all()
