@@ -43,7 +43,7 @@ using prism::DevBlock;
 static constexpr int CHAIN_COUNT_STRIDE = 64;
 /* d256 expert launches of at least this many 128-token tiles (two per CU)
  * use the 128-token kernel: each streamed weight fragment then feeds twice
- * the tokens. Smaller grids keep 64-token tiles (8 waves up to CU_COUNT tiles).
+ * the tokens. Smaller grids keep 64-token tiles (their waves: expert_w8).
  * A stage call of that size uses 96-token tiles of the same body instead:
  * alone on the GPU, its last round of workgroups is then less empty (batch 8
  * to 16 at 68x120: 7-13 % faster); inside the block chain the other

@@ -118,20 +118,23 @@ inline bool chain_attn_w8(const prism_model_desc& d, const ChainPlan& p, int64_t
 /* Experts, 64-token tiles: 8 waves? tiles: the launch's grid, n / 64 and a
  * partial tile per expert; n: its tokens; partial: the experts (0 if dense);
  * p: the chain's plan, NULL for a stage call.
- * At most one tile per CU: 8 waves per tile halve each wave's weight
- * stream; otherwise 4 waves x 2 tiles per CU. Alone on the GPU what counts
+ * Up to a tile per CU 8 waves per tile, which halve each wave's weight
+ * stream; more go as 4 waves x 2 tiles per CU. Where nothing runs beside the
+ * launch (a stage call, a chain without sub-chains) what counts
  * is the tiles that hold tokens, about half a tile per expert more than
- * n / 64 (the rest of the grid ends at once): n / 64 = 246, 16 experts
- * (254 tiles) 10.2 us on 8 waves, 11.1 on 4; 250 (258) 16.7 and 14.8; 64
- * experts 220 (252) 10.8 and 11.4; 236 (268) 17.1 and 15.3. Beside the other sub-chain's
- * attention a small second round costs less than slower tiles: a chain
- * with launches of 280 tiles 696 us on 8 waves, 770 on 4; of 296, 745 and
- * 789; of 320, 816 and 832 (or 807 and 789); of 352, 891 and 855. d128
+ * n / 64 (the rest of the grid ends at once): stage calls of n / 64 = 246, 16
+ * experts (254 tiles) 10.2 us on 8 waves, 11.1 on 4; 250 (258) 16.7 and 14.8;
+ * 64 experts 220 (252) 10.8 and 11.4; 236 (268) 17.1 and 15.3; a chain of one
+ * 120x128 frame, 64 experts (272) 580 and 542. Beside the other sub-chain's
+ * attention a small second round costs less than slower tiles, and the line
+ * lies at 5/4 of the grid's tiles per CU: chains with launches of 280 tiles
+ * 696 us on 8 waves, 770 on 4; of 296, 745 and 789; of 352, 891 and 855; at
+ * the line itself, 320, 816 and 832 on one run, 807 and 789 on another. d128
  * tiles leave room for two 8-wave workgroups per CU. */
 inline bool expert_w8(int dim, int64_t tiles, int64_t n, int partial, const ChainPlan* p) {
     if (dim != 256) return tiles < 2 * CU_COUNT;
     if (p && p->pair8) return true;
-    return !p ? (n + 63) / 64 + partial / 2 <= CU_COUNT : tiles <= CU_COUNT * 5 / 4;
+    return p && p->split > 1 ? tiles <= CU_COUNT * 5 / 4 : (n + 63) / 64 + partial / 2 <= CU_COUNT;
 }
 
 /* The leading blocks' expert weights are read past the memory-side cache

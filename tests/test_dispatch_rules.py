@@ -60,6 +60,10 @@ def test_attention_waves(rules):
     (32, 68, 120, 4, 4, 8), (16, 68, 120, 4, 4, 8), (16, 72, 120, 5, 4, 4),
     (64, 24, 64, 23, 8, 8), (64, 96, 120, 3, 4, 4),  # 264 and 288 | 180 and 360: unequal halves
     (64, 68, 120, 16, 4, 4),
+    # no sub-chains: filled tiles, n / 64 and half a tile per expert
+    (64, 112, 128, 1, 8, 8), (64, 114, 126, 1, 8, 4),  # 256 | 257
+    (16, 124, 128, 1, 8, 8), (16, 126, 126, 1, 8, 4),
+    (1, 128, 128, 1, 8, 8), (1, 130, 130, 1, 4, 4),    # a dense chain's last FFN
 ])
 def test_waves_of_routed_sub_chains(rules, experts, h, w, batch, attention, expert):
     assert rules.chain_attention_waves(256, experts, h, w, batch) == attention
