@@ -1,5 +1,7 @@
 """Shared test setup: import paths, the `gpu` marker and device fixtures."""
+import ctypes as C
 import os
+import subprocess
 import sys
 
 import numpy as np
@@ -14,6 +16,22 @@ for sub in ("prism-inference_amd", "oracle"):
 
 def pytest_configure(config):
     config.addinivalue_line("markers", "gpu: needs a HIP device (MI355X); runs through the C ABI")
+
+
+@pytest.fixture(scope="session")
+def rules(tmp_path_factory):
+    """The engine's dispatch rules (dispatch_rules.cpp over csrc/engine/rules.h)."""
+    so = str(tmp_path_factory.mktemp("rules") / "rules.so")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__",
+                    "-I", os.path.join(ROOT, "include"), os.path.join(ROOT, "tests", "dispatch_rules.cpp"), "-o", so],
+                   check=True, timeout=120)
+    lib = C.CDLL(so)
+    lib.attention_waves.argtypes = [C.c_int, C.c_longlong]
+    lib.projection_grid.argtypes, lib.projection_grid.restype = [C.c_int, C.c_longlong], C.c_longlong
+    lib.projection_waves.argtypes = [C.c_int, C.c_int, C.c_longlong]
+    lib.enc2_slots.argtypes = [C.c_longlong]
+    lib.grid_of.argtypes, lib.grid_of.restype = [C.c_longlong, C.c_int], C.c_uint
+    return lib
 
 
 @pytest.fixture(scope="session")

@@ -1,28 +1,8 @@
-"""Which kernels and grids the engine chooses, by size (csrc/engine/rules.h,
-compiled here into a small library): the edges of each rule."""
-import ctypes as C
-import os
-import subprocess
-
+"""Which kernels and grids the engine chooses, by size (csrc/engine/rules.h):
+the edges of each rule."""
 import pytest
 
-HERE = os.path.dirname(os.path.abspath(__file__))
 ONE = -1  # every block in one launch
-
-
-@pytest.fixture(scope="module")
-def rules(tmp_path_factory):
-    so = str(tmp_path_factory.mktemp("rules") / "rules.so")
-    subprocess.run(["g++", "-std=c++17", "-O1", "-shared", "-fPIC", "-D__HIP_PLATFORM_AMD__",
-                    "-I", os.path.join(HERE, "..", "include"), os.path.join(HERE, "dispatch_rules.cpp"), "-o", so],
-                   check=True, timeout=120)
-    lib = C.CDLL(so)
-    lib.attention_waves.argtypes = [C.c_int, C.c_longlong]
-    lib.projection_grid.argtypes, lib.projection_grid.restype = [C.c_int, C.c_longlong], C.c_longlong
-    lib.projection_waves.argtypes = [C.c_int, C.c_int, C.c_longlong]
-    lib.enc2_slots.argtypes = [C.c_longlong]
-    lib.grid_of.argtypes, lib.grid_of.restype = [C.c_longlong, C.c_int], C.c_uint
-    return lib
 
 
 @pytest.mark.parametrize("dim,experts,h,w,batch,plan", [

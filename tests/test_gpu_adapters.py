@@ -150,11 +150,17 @@ def test_adapted_chain(hip, engine, device_arena, name, nb, H, W, batch, affine)
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,nb,H,W,batch,affine", [
-    ("moe16", 2, 20, 28, 4, False),    # two sub-chains; ragged windows
+    ("moe16", 2, 20, 28, 4, False),    # ragged windows
+    ("moe16", 2, 20, 28, 17, False),   # 204 windows: two sub-chains
     ("moe64", 1, 68, 120, 1, False),   # one block: up- and down-projection in the same block
     ("moe64", 3, 68, 120, 1, False),   # 8-wave kernels
     ("dense128", 3, 68, 120, 2, False),
-    ("std256", 2, 16, 16, 5, False),   # dense d256, sub-chains of 2 and 3 frames
+    ("std256", 2, 16, 16, 5, False),   # dense d256
+    ("std256", 2, 17, 25, 23, False),  # 276 windows: dense sub-chains of 11 and 12 frames
+    # from 3 blocks on all but the last run in one launch, its up-projection first
+    ("std256", 4, 20, 28, 3, True),    # 8 waves
+    ("std256", 3, 60, 90, 5, True),    # 480 windows: 4 waves; padded-slot and HALF+padded bodies
+    ("dense128", 4, 60, 90, 8, True),  # 768 windows: d128, 4 waves
     # LN affines (LN1 beta != 0): block 0's windows with padded slots run the
     # PAD / PAD+HALF bodies with the fused up-projection; every window of
     # every block equals the separate calls bit for bit

@@ -7,8 +7,8 @@ the C ABI, against the oracle.
   batch 16) against the free-running oracle. Near-tie routing flips move a few tokens by more than the per-block
   bound, so the whole-model check bounds the mean error (2e-3) and the share
   of tokens moved by more than 2e-2 (2 %).
-- Teacher-forced through the chain's own kernels: the chain runs a batch of 4
-  or more frames as two sub-chains of half the frames each, and every MoE block
+- Teacher-forced through the chain's own kernels: the chain runs a batch of
+  more than 192 windows as two sub-chains of half the frames each, and every MoE block
   as one routed attention launch (prism_attn_route) plus one grouped expert
   launch (prism_experts). Calling those two entry points on half the batch
   runs the chain's attention kernels (same grid, same variant) and its expert
@@ -36,22 +36,22 @@ def f16(bits):
     return O.f16bits_to_f32(bits)
 
 
-def subchain_batches(batch):
-    """Frames per sub-chain, as the engine splits a batch (2 sub-chains from 4
-    frames on)."""
-    if batch < 4:
+def subchain_batches(rules, cfg, batch):
+    """Frames per sub-chain, as the engine splits a batch."""
+    if abs(rules.chain(cfg.dim, cfg.n_experts, cfg.H, cfg.W, batch)) < 2:
         return [batch]
     return [batch // 2, batch - batch // 2]
 
 
-def attn_kernel(dim, n_experts, windows, chain=False):
-    """The attention kernel the engine launches for a grid of `windows`
-    workgroups: 8 waves below 512 windows, 4 waves from 512 on; _r<k> routes
-    over 16k padded experts; _ffn: a dense block of the chain, its FFN in the
-    same launch."""
-    npt = (n_experts + 15) // 16 if n_experts > 1 else 0
-    return (f"prism_attn_d{dim}{'_w8' if windows < 512 else ''}{f'_r{npt}' if npt else ''}"
-            + ("_ffn" if chain and not npt else ""))
+def attn_kernel(rules, cfg, batch):
+    """The attention kernel of the engine's chain: _r<k> routes over 16k padded
+    experts; _ffn: a dense block with its FFN in the same launch; chain: all of
+    a dense chain's blocks."""
+    plan = rules.chain(cfg.dim, cfg.n_experts, cfg.H, cfg.W, batch)
+    w8 = "_w8" if rules.chain_attention_waves(cfg.dim, cfg.n_experts, cfg.H, cfg.W, batch) == 8 else ""
+    if cfg.n_experts > 1:
+        return f"prism_attn_d{cfg.dim}{w8}_r{(cfg.n_experts + 15) // 16}"
+    return f"prism_chain_d{cfg.dim}{w8}" if plan < 0 else f"prism_attn_d{cfg.dim}{w8}_ffn"
 
 
 @pytest.mark.gpu
@@ -59,14 +59,14 @@ def attn_kernel(dim, n_experts, windows, chain=False):
     ("moe32", 4, "prism_attn_d256_r2"),   # 2 x 2 frames of 510 windows: the 4-wave N=32 kernel
     ("moe16", 1, "prism_attn_d256_w8_r1"),
     ("moe64", 16, "prism_attn_d256_r4"),  # the headline step: 2 x 8 frames, 1080 windows each
-    ("dense128", 16, "prism_attn_d128_ffn"),  # 2 x 8 frames of 1080 windows, FFN in the launch
+    ("dense128", 16, "prism_chain_d128"),     # 2,160 windows, every block in one launch
     ("std256", 16, "prism_attn_d256_ffn"),    # 2 x 8 frames, FFN in the launch
+    ("std256", 1, "prism_chain_d256_w8"),
 ])
-def test_config_chain_against_oracle(hip, engine, device_arena, name, batch, kernel):
+def test_config_chain_against_oracle(hip, engine, rules, device_arena, name, batch, kernel):
     cfg = P.CONFIGS[name]
     H, W, nb = cfg.H, cfg.W, cfg.n_blocks
-    windows = ((H + 7) // 8) * ((W + 7) // 8)
-    assert attn_kernel(cfg.dim, cfg.n_experts, windows * subchain_batches(batch)[0], chain=True) == kernel
+    assert attn_kernel(rules, cfg, batch) == kernel
     desc = cfg.desc()
     blob, offs = P.synth_weights(desc, seed=0, routing=cfg.routing)
     engine.load_weights(desc, blob, offs)
@@ -104,7 +104,7 @@ def test_config_chain_against_oracle(hip, engine, device_arena, name, batch, ker
     ("moe32", 2, 4),    # sub-chains of 2 frames at 135x240: 1020-window prism_attn_d256_r2
     ("moe64", 16, 1),   # every block of the headline model at batch 1 (8-wave kernels)
 ])
-def test_chain_kernels_teacher_forced(hip, engine, device_arena, name, nb, batch):
+def test_chain_kernels_teacher_forced(hip, engine, rules, device_arena, name, nb, batch):
     cfg = P.CONFIGS[name]
     H, W, N, d = cfg.H, cfg.W, cfg.n_experts, cfg.dim
     T = H * W
@@ -117,7 +117,7 @@ def test_chain_kernels_teacher_forced(hip, engine, device_arena, name, nb, batch
     for b in range(nb):
         nxt = np.empty_like(cur)
         f0 = 0
-        for sb in subchain_batches(batch):
+        for sb in subchain_batches(rules, cfg, batch):
             n = sb * T
             c = O.cfg(d, cfg.n_heads, cfg.head_dim, N, H, W, sb, True)
             xin = cur[f0 * T:(f0 + sb) * T]
@@ -129,7 +129,7 @@ def test_chain_kernels_teacher_forced(hip, engine, device_arena, name, nb, batch
             pa = engine.attn_push(b, 0, n * d)
             pr = engine.router_push(b, T, n * d, 0, n, n + N)
             print(f"[tf] {name} block {b} frames {f0}..{f0 + sb - 1} "
-                  f"({attn_kernel(d, N, sb * ((H + 7) // 8) * ((W + 7) // 8))})", flush=True)
+                  f"({attn_kernel(rules, cfg, batch)})", flush=True)
             assert engine.attn_route(pa, pr, feats.ptr, aux.ptr, sb) == 0, engine.error()
             hip.sync()
             h_gpu = f16(hip.download(np.empty(n * d, np.uint16), feats.ptr + n * d * 2)).reshape(n, d)

@@ -75,8 +75,9 @@ EXTRA = {
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,nb,H,W,batch", [
     ("moe64", 3, 68, 120, 1),      # 8-wave routed kernel, 4 router row tiles
-    ("moe64", 2, 68, 120, 4),      # two sub-chains of 2 frames (270 windows each): 8-wave kernels
+    ("moe64", 2, 68, 120, 4),      # two sub-chains of 2 frames (270 windows each), both on 8 waves
     ("moe16", 2, 20, 28, 3),       # 1 row tile, ragged windows, 3 frames (one chain)
+    ("moe16", 2, 20, 28, 17),      # two sub-chains of 8 and 9 frames
     ("moe16", 1, 20, 28, 2),       # one block: its counters are cleared inside the chain
     ("moe40", 2, 68, 120, 1),
     ("moe40", 2, 68, 120, 4),
@@ -86,7 +87,7 @@ EXTRA = {
                                    # blocks' expert weights stream non-temporally in the chain
     ("moe64", 2, 68, 120, 16),     # sub-chains of 8 frames: 4-wave _r4, 128-token expert tiles
                                    # (the stage calls: 96-token tiles of the same body)
-    ("moe32", 2, 135, 240, 1),     # 510 windows, 8 waves, 2 router row tiles split over wave pairs
+    ("moe32", 2, 135, 240, 1),     # 510 windows: 4 waves, 2 router row tiles
     ("moe32", 2, 135, 240, 4),     # sub-chains of 2 frames (1020 windows each): 4-wave _r2
     ("moe16", 2, 68, 120, 8),      # sub-chains of 4 frames (540 windows each): 4-wave _r1
     ("moe40", 2, 68, 120, 8),      # 4-wave _r3
@@ -137,16 +138,20 @@ def test_chain_matches_stage_calls(hip, engine, device_arena, name, nb, H, W, ba
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,nb,H,W,batch,affine", [
-    ("dense128", 3, 68, 120, 1, False),   # 8-wave fused kernel; the bottom windows hold 4 rows
-    ("dense128", 2, 68, 120, 16, False),  # sub-chains of 8 frames: 4-wave fused kernel
+    ("dense128", 3, 68, 120, 1, False),   # one launch, 8 waves; the bottom windows hold 4 rows
+    ("dense128", 2, 68, 120, 16, False),  # one launch, 4 waves
+    ("dense128", 1, 68, 120, 1, True),    # one block: the fused attention + FFN kernels, 8 waves
+    ("dense128", 1, 60, 90, 16, True),    # ... 4 waves
     ("dense128", 2, 60, 90, 4, True),     # ragged windows on both edges with LN1 beta != 0
                                           # (the padded-slot bodies), LN2 affine folded into W1
     ("dense128", 2, 68, 120, 1, True),
-    ("dense128", 2, 60, 90, 16, True),    # 4-wave fused kernel (768 windows per sub-chain) on the
-                                          # padded-slot and HALF+padded bodies
-    ("std256", 2, 68, 120, 2, False),     # d256, 8-wave fused kernel (270 windows)
+    ("dense128", 2, 60, 90, 16, True),    # 4 waves (1,536 windows) on the padded-slot and
+                                          # HALF+padded bodies
+    ("std256", 2, 68, 120, 2, False),     # d256, one launch, 4 waves (270 windows)
+    ("std256", 3, 60, 90, 5, True),       # ... 480 windows, padded-slot and HALF+padded bodies
+    ("std256", 2, 17, 25, 23, True),      # 276 windows: sub-chains of 8-wave fused launches
     ("std256", 2, 68, 120, 1, True),
-    ("std256", 2, 68, 120, 16, False),    # 1080 windows per sub-chain: 4-wave fused kernel
+    ("std256", 2, 68, 120, 16, False),    # 1,080 windows per sub-chain: 4-wave fused launches
     ("std256", 2, 60, 90, 16, True),      # 4-wave, padded-slot and HALF+padded bodies
 ])
 def test_dense_chain_matches_stage_calls(hip, engine, device_arena, name, nb, H, W, batch, affine):

@@ -67,8 +67,10 @@ def _reference(hip, device_arena, name, nb, H, W, batch, adapted, x):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("name,nb,H,W,batch,adapted", [
-    ("moe16", 2, 20, 28, 3, False),   # 3 frames: one chain (sub-chains start at 4 frames)
-    ("moe16", 2, 20, 28, 5, False),   # two sub-chains (2 + 3 frames)
+    ("moe16", 2, 20, 28, 3, False),   # 36 windows: one chain
+    ("moe16", 2, 20, 28, 5, False),
+    ("moe16", 2, 20, 28, 17, False),  # 204 windows: two sub-chains (8 + 9 frames)
+    ("std256", 2, 17, 25, 23, False),  # 276: two dense sub-chains
     ("moe64", 2, 68, 120, 1, True),   # the adapted chain: 128-channel in/out
     ("dense128", 2, 68, 120, 4, False),
 ])

@@ -240,10 +240,10 @@ FUSED_EXTRA = {
 
 def attn_kernel(dim, n_experts, windows):
     """The attention kernel the engine launches for `windows` workgroups
-    (engine.cpp enqueue_attn): 8 waves below 512 windows, 4 waves from 512 on;
-    _r<k> routes over 16k padded experts."""
+    (a stage call): 8 waves up to 256 windows at d256, 511 at d128, 4 waves
+    above; _r<k> routes over 16k padded experts."""
     npt = (n_experts + 15) // 16 if n_experts > 1 else 0
-    return f"prism_attn_d{dim}{'_w8' if windows < 512 else ''}{f'_r{npt}' if npt else ''}"
+    return f"prism_attn_d{dim}{'_w8' if windows <= (256 if dim == 256 else 511) else ''}{f'_r{npt}' if npt else ''}"
 
 
 @pytest.mark.gpu
@@ -252,6 +252,8 @@ def attn_kernel(dim, n_experts, windows):
     ("moe64", 68, 120, 4, "prism_attn_d256_r4"),       # 540 windows
     ("moe64", 68, 120, 16, "prism_attn_d256_r4"),      # the headline batch: 2,160 windows
     ("moe16", 9, 13, 1, "prism_attn_d256_w8_r1"),      # one row tile, ragged windows
+    ("moe16", 61, 127, 2, "prism_attn_d256_w8_r1"),    # 256 windows
+    ("moe16", 8, 2051, 1, "prism_attn_d256_r1"),       # 257
     ("moe40", 68, 120, 1, "prism_attn_d256_w8_r3"),    # 3 row tiles, 24 padded experts
     ("moe24d128", 68, 120, 2, "prism_attn_d128_w8_r2"),
     ("moe16", 68, 120, 4, "prism_attn_d256_r1"),

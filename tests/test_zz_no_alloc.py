@@ -27,8 +27,11 @@ def workspace_bytes(desc, batch):
             + up(2 * desc.n_blocks * desc.n_experts * 64 * 4) + up(desc.n_experts * n * 4))
 
 
+SPLIT_BATCH = 17  # frames of 20x28: 204 windows, two sub-chains of a MoE chain
+
+
 @pytest.mark.gpu
-def test_forward_noalloc_equals_forward(hip, device_arena):
+def test_forward_noalloc_equals_forward(hip, rules, device_arena):
     eng = P.Engine(0)   # a fresh context: prism_forward_noalloc runs before it has any workspace
     try:
         cfg = P.CONFIGS["moe64"]
@@ -38,7 +41,8 @@ def test_forward_noalloc_equals_forward(hip, device_arena):
         eng.load_weights(desc, blob, offs)
         d = cfg.dim
         results = {}
-        for batch in (5, 2):    # two sub-chains, then one smaller chain
+        assert [rules.chain(d, 64, H, W, b) for b in (SPLIT_BATCH, 5)] == [2, 1]
+        for batch in (SPLIT_BATCH, 5):    # two sub-chains, then one smaller chain
             n = batch * H * W
             assert workspace_bytes(desc, batch) <= SCRATCH_BYTES
             x = P.synth_features(cfg, batch=batch, H=H, W=W, seed=20 + batch).reshape(-1)
@@ -113,12 +117,13 @@ def _model(seed=4, nb=3, H=20, W=28):
 
 
 @pytest.mark.gpu
-def test_forward_noalloc_two_contexts_two_streams(hip, device_arena):
+def test_forward_noalloc_two_contexts_two_streams(hip, rules, device_arena):
     """Two contexts on one GPU, each on its own stream, enqueue four calls each
     with no synchronisation in between: the calls share the scratch array and
     must run one after another, so every output equals prism_forward's."""
     cfg, desc, blob, offs = _model()
-    H, W, batch, d = desc.spatial_h, desc.spatial_w, 5, cfg.dim
+    H, W, batch, d = desc.spatial_h, desc.spatial_w, SPLIT_BATCH, cfg.dim
+    assert rules.chain(d, 64, H, W, batch) == 2
     n = batch * H * W
     engs = [P.Engine(0), P.Engine(0)]
     try:
@@ -152,14 +157,15 @@ def test_forward_noalloc_two_contexts_two_streams(hip, device_arena):
 
 
 @pytest.mark.gpu
-def test_forward_noalloc_under_global_capture(hip, device_arena):
+def test_forward_noalloc_under_global_capture(hip, rules, device_arena):
     """The call inside hipStreamCaptureModeGlobal capture (an allocation or a
     device synchronisation during it would invalidate the capture): the graph
     replays three times, with eager calls of the same entry point and
     synchronisations between the replays, and every replay equals
     prism_forward."""
     cfg, desc, blob, offs = _model(seed=6)
-    H, W, batch, d = desc.spatial_h, desc.spatial_w, 4, cfg.dim
+    H, W, batch, d = desc.spatial_h, desc.spatial_w, SPLIT_BATCH, cfg.dim
+    assert rules.chain(d, 64, H, W, batch) == 2  # the capture forks and joins
     n = batch * H * W
     eng = P.Engine(0)
     try:
