@@ -1,8 +1,6 @@
-"""The chain's choice of kernels and sub-chains by the number of windows: 8-wave
-workgroups up to one per CU (256 windows at d256, 511 at d128),
-4-wave ones above; two sub-chains above 192 windows (MoE) or 512 (dense); a
-dense chain in one launch (d128, and up to 512 windows at d256). Frames never interact, so a frame's
-output is the same bits whichever side of an edge its batch lies on."""
+"""The chain's choice of kernels and sub-chains by the number of windows (the
+rules' edges: test_dispatch_rules.py). Frames never interact, so a frame's output is
+the same bits whichever side of an edge its batch lies on."""
 import numpy as np
 import pytest
 
@@ -13,7 +11,7 @@ import prism_amd as P
 @pytest.mark.parametrize("name,batches", [
     ("moe64", (1, 3, 4, 5, 9)),     # 64, 192 | 256 windows; a sub-chain of 256, of 320
     ("moe32", (1, 3, 4, 9)),
-    ("std256", (1, 4, 5, 8, 9)),
+    ("std256", (1, 4, 5, 6, 8, 9)),  # 256 | 320 in 8-wave sub-chains | 384, 512 | 576 in 4-wave ones
     ("dense128", (1, 7, 8, 9)),     # 448 | 512 | 576
 ])
 def test_frame_is_the_same_in_every_batch(hip, engine, device_arena, name, batches):
@@ -26,7 +24,12 @@ def test_frame_is_the_same_in_every_batch(hip, engine, device_arena, name, batch
     x = P.synth_features(cfg, batch=max(batches), H=H, W=W, seed=6).reshape(max(batches), n * d)
     dx, dy = device_arena(x.nbytes), device_arena(x.nbytes)
     hip.upload(dx.ptr, x)
-    ref = None
+    ref = []  # every frame on its own
+    for f in range(max(batches)):
+        engine.forward(dx.ptr + f * n * d * 2, dy.ptr, 1)
+        hip.sync()
+        ref.append(hip.download(np.empty(n * d, np.uint16), dy.ptr))
+    assert all((ref[0] != r).any() for r in ref[1:])
     for b in batches:
         for graph in (False, True):
             print(f"[dispatch] {name} batch {b} graph {graph}", flush=True)
@@ -34,13 +37,37 @@ def test_frame_is_the_same_in_every_batch(hip, engine, device_arena, name, batch
             engine.forward(dx.ptr, dy.ptr, b, graph=graph)
             hip.sync()
             y = hip.download(np.empty((b, n * d), np.uint16), dy.ptr)
-            if ref is None:
-                ref = y
-            assert (y[0] == ref[0]).all(), f"batch {b}: frame 0 differs"
-            if b == max(batches):  # the last frame (of the second sub-chain) on its own
-                engine.forward(dx.ptr + (b - 1) * n * d * 2, dy.ptr, 1, graph=graph)
-                hip.sync()
-                assert (hip.download(np.empty(n * d, np.uint16), dy.ptr) == y[b - 1]).all()
+            for f in range(b):
+                assert (y[f] == ref[f]).all(), f"batch {b}: frame {f} differs"
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,H,W,batch", [
+    ("moe64", 24, 64, 22),   # 528 windows, more than 32 experts: both sub-chains on 8 waves
+    ("moe64", 24, 64, 23),   # ... of 264 and 288
+    ("moe64", 17, 25, 48),   # 576 windows, few tokens: by their own windows
+    ("std256", 17, 25, 23),  # 276 windows, a third of them half padded: sub-chains
+    ("std256", 9, 24, 43),   # 258, the last two half padded: one launch
+])
+def test_small_frames_in_a_large_batch(hip, engine, device_arena, name, H, W, batch):
+    """First, middle (the sub-chains' seam) and last frames as on their own."""
+    cfg = P.CONFIGS[name]
+    desc = cfg.desc(n_blocks=2, H=H, W=W)
+    blob, offs = P.synth_weights(desc, seed=5, routing=cfg.routing)
+    engine.load_weights(desc, blob, offs)
+    d, n = cfg.dim, H * W
+    x = P.synth_features(cfg, batch=batch, H=H, W=W, seed=6).reshape(batch, n * d)
+    dx, dy, dz = device_arena(x.nbytes), device_arena(x.nbytes), device_arena(n * d * 2)
+    hip.upload(dx.ptr, x)
+    print(f"[dispatch] {name} {H}x{W} batch {batch}", flush=True)
+    hip.memset(dy.ptr, 0xFF, x.nbytes)
+    engine.forward(dx.ptr, dy.ptr, batch)
+    hip.sync()
+    y = hip.download(np.empty((batch, n * d), np.uint16), dy.ptr)
+    for f in sorted({0, 1, batch // 2 - 1, batch // 2, batch // 2 + 1, batch - 2, batch - 1}):
+        engine.forward(dx.ptr + f * n * d * 2, dz.ptr, 1)
+        hip.sync()
+        assert (y[f] == hip.download(np.empty(n * d, np.uint16), dz.ptr)).all(), f"frame {f} differs"
 
 
 @pytest.mark.gpu
@@ -113,7 +140,8 @@ def test_stage_counts_by_the_last_workgroup(hip, engine, device_arena, name, H, 
 @pytest.mark.parametrize("name,W", [("moe16", 248), ("moe16", 249), ("moe64", 224), ("moe64", 225)])
 def test_expert_stage_at_the_edge_of_one_round(hip, engine, device_arena, name, W):
     """n / 64 + n_experts / 2 = 256 tiles (8 waves) and 257 (4 waves): a frame's
-    rows are the same bits alone and in a batch of two (4 waves)."""
+    rows are the same bits alone, in a batch of two (4 waves), and its first quarter's
+    alone (8 waves)."""
     H, d = 64, P.CONFIGS[name].dim
     cfg = P.CONFIGS[name]
     desc = cfg.desc(n_blocks=1, H=H, W=W)
@@ -123,16 +151,19 @@ def test_expert_stage_at_the_edge_of_one_round(hip, engine, device_arena, name, 
     x = P.synth_features(cfg, batch=2, H=H, W=W, seed=12).reshape(-1)
     feats, aux = device_arena(2 * x.nbytes), device_arena(P.aux_elems(N, 2 * T) * 4)
     ys = []
-    for batch in (1, 2):
+    for batch, T in ((1, H * W), (2, H * W), (1, H * W // 4)):
         n = batch * T
         hip.upload(feats.ptr, x)
+        hip.memset(feats.ptr + x.nbytes, 0xFF, x.nbytes)  # NaN: every row must be written
         print(f"[dispatch] experts {name} {H}x{W} batch {batch}", flush=True)
         assert engine.router(engine.router_push(0, T, 0, 0, n, n + N), feats.ptr, aux.ptr, batch) == 0, engine.error()
-        push = engine.expert_push(0, T, 0, 2 * T * d, 0, n, n + N)
+        push = engine.expert_push(0, T, 0, x.size, 0, n, n + N)
         assert engine.experts(push, feats.ptr, aux.ptr, batch) == 0, engine.error()
         hip.sync()
-        ys.append(hip.download(np.empty(T * d, np.uint16), feats.ptr + x.nbytes))
-    assert (ys[0] == ys[1]).all()
+        ys.append(hip.download(np.empty(n * d, np.uint16), feats.ptr + x.nbytes))
+    frame = H * W * d
+    assert (ys[0] == ys[1][:frame]).all() and (ys[2] == ys[0][:frame // 4]).all()
+    assert np.isfinite(ys[1].view(np.float16)).all()
 
 
 @pytest.mark.gpu
