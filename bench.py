@@ -390,7 +390,7 @@ def main():
         r_push = eng.router_push(0, T, n * d, 0, n, n + N)
         e_push = eng.expert_push(0, T, n * d, 0, 0, n, n + N)
         # the chain's MoE-block kernel: attention + routing in one launch (plus
-        # the one-workgroup counter clear the stage call issues before it)
+        # what the stage call does beyond the chain's launch: its last workgroup moves the counts)
         rr_push = eng.router_push(0, T, n * d, 0, n, n + N)
         t_route = time_stage(hip, lambda: eng.attn_route(a_push, rr_push, feats, aux, B, stream), args.stage_reps,
                              stream)
@@ -398,7 +398,7 @@ def main():
         t_router = time_stage(hip, lambda: eng.router(r_push, feats, aux, B, stream), args.stage_reps, stream)
         t_expert = time_stage(hip, lambda: eng.experts(e_push, feats, aux, B, stream), args.stage_reps, stream)
         kname += f"_r{(N + 15) // 16}"
-        timed = "prism_attn_route stage call: the routed attention kernel + its 1-workgroup count copy"
+        timed = "prism_attn_route stage call: the routed attention kernel, its last workgroup moving the counts"
     else:
         # dense blocks: attention, then the FFN as the expert stage with one expert
         e_push = eng.expert_push(0, T, n * d, 0)

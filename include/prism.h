@@ -92,8 +92,8 @@ typedef struct prism_attn_push {
  * counts [n_experts] (tokens per expert), and perm [n_experts][batch*n_tokens]
  * (token indices bucketed by expert: the counting sort's output; the order
  * inside a bucket is unspecified). The call writes the counts itself (the
- * router kernel counts into a row of the context's own, then a one-workgroup
- * launch copies the totals), so nothing is required of them on entry. */
+ * router kernel counts into a row of the context's own, and its last workgroup
+ * moves the totals), so nothing is required of them on entry. */
 typedef struct prism_router_push {
     int32_t n_tokens, dim, n_experts;
     int64_t router_w, router_b;
@@ -186,8 +186,8 @@ int prism_load_weights_file(prism_ctx* ctx, const prism_model_desc* desc,
 /* features: device fp16 arena; aux: device int32 arena. The weight offsets
  * in the push structs must name tensors of a loaded block. prism_router
  * writes the assignment, the counts (from zero) and the buckets; it counts
- * into a row of the context's own, counters 256 bytes apart, and a
- * one-workgroup launch copies the totals to `counts`, so router and
+ * into a row of the context's own, counters 256 bytes apart, and the
+ * launch's last workgroup moves the totals to `counts`, so router and
  * attention-route calls on one context must not overlap on different
  * streams. */
 int prism_attn(prism_ctx* ctx, const prism_attn_push* p, void* features, int32_t batch,
@@ -207,7 +207,7 @@ int prism_experts(prism_ctx* ctx, const prism_expert_push* p, void* features,
  * ids and counts; the order inside a bucket is unspecified). No reference
  * counterpart as a single call: the block chain uses it for MoE blocks. The
  * kernel counts into a row of the context's own, counters 256 bytes apart,
- * and a one-workgroup launch copies the totals to `counts`: calls on one
+ * and the launch's last workgroup moves the totals to `counts`: calls on one
  * context must not overlap on different streams. */
 int prism_attn_route(prism_ctx* ctx, const prism_attn_push* pa, const prism_router_push* pr,
                      void* features, int32_t* aux, int32_t batch, void* stream);

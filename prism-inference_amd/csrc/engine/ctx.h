@@ -118,8 +118,8 @@ struct prism_ctx {
     void* scratch = nullptr;      /* this device's allocation-free workspace (scratch.hip) */
     bool counts_dirty = false;    /* block 0's counters may be nonzero */
     unsigned last_grid = 0;       /* workgroups of the last kernel launched (chain timing) */
-    int32_t* stage_counts = nullptr; /* prism_attn_route: private counters, CHAIN_COUNT_STRIDE apart */
-    bool stage_dirty = false;        /* ... possibly nonzero (a call stopped between its launches) */
+    int32_t* stage_counts = nullptr; /* routing stage calls: private counters, CHAIN_COUNT_STRIDE apart, then the tickets */
+    bool stage_dirty = false;        /* ... possibly nonzero (a launch that failed) */
 
     hipStream_t user_stream = nullptr;  /* prism_init_with_device: the renderer's stream */
     hipEvent_t ev_t0 = nullptr, ev_t1 = nullptr; /* prism_infer_gpu timing */

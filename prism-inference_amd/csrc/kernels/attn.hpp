@@ -887,8 +887,8 @@ PRISM_ATTN_KERNELS(128, 16, 2, _r2)
 PRISM_ATTN_KERNELS(128, 16, 3, _r3)
 PRISM_ATTN_KERNELS(128, 16, 4, _r4)
 
-/* dense blocks in the chain: attention with the block's FFN fused (the
- * chain's one launch per dense block) */
+/* one dense block: attention with its FFN fused (the launches of sub-chains,
+ * of one-block models and of two-block models with the adapters fused) */
 extern "C" __global__ void __launch_bounds__(256, 2) prism_attn_d128_ffn(AttnArgs a) {
     __shared__ AttnLds<128, 0> lds;
     attn_window<128, 16, 4, 0, true>(a, lds);
@@ -907,7 +907,9 @@ extern "C" __global__ void __launch_bounds__(512, 1) prism_attn_d256_w8_ffn(Attn
 }
 /* a whole dense chain in one launch: windows are never shifted, so a window's
  * 64 tokens meet no others in any block, and its rows stay in LDS from the
- * first block's input to the last one's output */
+ * first block's input to the last one's output. The block loop's parameter
+ * pointers spill SGPRs to VGPR lanes (d256 4 waves 509, 8 waves 76; d128 4
+ * waves 30), none to scratch. */
 extern "C" __global__ void __launch_bounds__(512, 4) prism_chain_d128_w8(AttnArgs a) {
     __shared__ AttnLds<128, 0> lds;
     attn_window<128, 16, 8, 0, true, true>(a, lds);

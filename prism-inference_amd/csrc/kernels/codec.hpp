@@ -307,7 +307,9 @@ __device__ __forceinline__ void codec_dec_out(const CodecArgs& a) {
  * k = 32 ky + 10 kx + ic, 3 k-steps (the host packs W's stored column ic * 9 +
  * tap there, zeros elsewhere). The odd dword stride (5) keeps the reads of 16
  * consecutive pixels free of bank conflicts. (9 taps x 16 halfs a pixel, 5
- * k-steps, read 1.7 times the LDS bytes, which bound the fused launch.) */
+ * k-steps, read 1.7 times the LDS bytes, which bound the fused launch; the
+ * sums of the two differ in their last bits, their error against 64 bits does
+ * not: 3.9e-4 over the encoder.) */
 static constexpr int ENC0_CP = 10, ENC0_KS = 3;
 typedef unsigned u4 __attribute__((ext_vector_type(4)));
 typedef unsigned u2 __attribute__((ext_vector_type(2)));

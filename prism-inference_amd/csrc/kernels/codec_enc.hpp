@@ -10,7 +10,7 @@
  * 2 x1 - 1 .. 2 x1 + 63, a 9 x 65 region, whose own taps need the 11 x 67
  * frame window around it. The window goes into LDS as in enc0, enc0 of the
  * region into a second LDS array (the same fragments, k order, rounding and
- * ReLU as prism_codec_enc0; zeros where it leaves the map; the halo row and
+ * ReLU as the stage kernel prism_codec_enc0; zeros where it leaves the map; the halo row and
  * column, 12 % of the region, are the neighbours' too), the block's own 8 x 64
  * e0 pixels from there to the e0 map (the decoder's skip) as whole rows, and
  * enc1 reads its taps from that array (k = tap * 32 + ic, as
@@ -234,8 +234,9 @@ extern "C" __global__ void __launch_bounds__(512, 4) prism_codec_enc01(CodecArgs
  * fragments DW k-steps ahead: no input pixel or weight fragment is fetched by
  * more than one wave of the workgroup. The output tile leaves as whole pixels.
  * Persistent over one XCD's band of blocks; the next block's window is
- * requested before this block's end. 128 VGPRs, two workgroups per CU. enc2 +
- * enc3 at 960x540 9.8 + 6.8 us, at 1920x1080 29 + 22 (one fused launch of 8
+ * requested before this block's end. 128 VGPRs, two workgroups fit a CU (enc2
+ * launches one up to four blocks per CU: codec_enc2_slots). enc2 + enc3 at
+ * 960x540 9.0 + 6.8 us, at 1920x1080 29 + 22 (one fused launch of 8
  * waves per CU, enc2 recomputing its halo: 19.6 and 80). Without the operand
  * reads enc3 would be 20 % faster, without its weights 7 %. Blocks of 8 x 8
  * for enc3 (half the weight bytes): 22 against 23.7 us at 1920x1080, 5 %
