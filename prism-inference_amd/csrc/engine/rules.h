@@ -40,7 +40,13 @@ struct ChainPlan {
  * one half's attention launch no longer fits beside the other's experts for
  * free: 16 blocks, one chain against two: 160 windows 411 and 418 us, 192
  * 442 and 438, 256 578 and 509 (64 experts), 270 641 and 504, 288 684 and
- * 539, 504 859 and 814. A dense block is one launch: its frames stay together
+ * 539, 504 859 and 814. With more than 32 experts, whose weights fill most of
+ * a small launch's time, not while both launches are one round of 8-wave
+ * workgroups (expert_w8): 64 experts, graphs of three frames of 56x75 (210
+ * windows) 451 and 480 us, of 36x123 (240) 457 and 482, of two of 81x81 462
+ * and 479, of 9 of 24x64 (216) 466 and 483, of 6 of 33x51 (210) 419 and 440
+ * (eager, where the second stream costs less, 441 and 437, 446 and 434, 450 and
+ * 462, 455 and 455, 409 and 410). A dense block is one launch: its frames stay together
  * while they fit one round of the 4-wave kernels (two workgroups per CU; four
  * blocks, 256 windows 83 and 91 us, d128 512 windows 61 and 74; 540 windows
  * 170 and 150).
@@ -83,8 +89,10 @@ constexpr int CHAIN_PAIR8_MAX = CU_COUNT * 11 / 5, CHAIN_PAIR8_TILES = CU_COUNT 
 inline ChainPlan chain_plan(const prism_model_desc& d, int batch) {
     const int64_t wx = (d.spatial_w + 7) / 8, frame = wx * ((d.spatial_h + 7) / 8), windows = frame * batch;
     if (d.n_experts > 1) {
-        const int split = windows > CHAIN_SPLIT_ROUTED ? std::min(CHAIN_SPLIT, batch) : 1;
         const int64_t tokens = (int64_t)d.spatial_w * d.spatial_h * batch;
+        const bool one_round = d.dim == 256 && d.n_experts > 32 && windows <= CU_COUNT &&
+                               (tokens + 63) / 64 + d.n_experts / 2 <= CU_COUNT;
+        const int split = windows > CHAIN_SPLIT_ROUTED && !one_round ? std::min(CHAIN_SPLIT, batch) : 1;
         const bool pair8 = split > 1 && d.dim == 256 && d.n_experts > 32 && windows > 2 * CU_COUNT &&
                            windows <= CHAIN_PAIR8_MAX && (batch + 1) / 2 * frame <= CU_COUNT * 9 / 8 &&
                            tokens / 128 + d.n_experts > CHAIN_PAIR8_TILES;

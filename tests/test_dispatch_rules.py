@@ -8,6 +8,10 @@ ONE = -1  # every block in one launch
 @pytest.mark.parametrize("dim,experts,h,w,batch,plan", [
     (256, 64, 64, 64, 3, 1), (256, 64, 64, 64, 4, 2),      # 192 | 256 windows
     (256, 16, 135, 240, 1, 1),                             # one frame never splits
+    # more than 32 experts: not while windows and filled tiles are one round
+    (256, 64, 56, 75, 3, 1), (256, 32, 56, 75, 3, 2),      # 210 windows, 229 tiles
+    (256, 64, 56, 128, 2, 1), (256, 64, 57, 128, 2, 2),    # 256 tiles | 260
+    (256, 64, 17, 25, 21, 1), (256, 64, 17, 25, 22, 2),    # 252 | 264 windows
     (128, 1, 68, 120, 1, ONE), (128, 1, 68, 120, 16, ONE),  # d128: always together
     (256, 1, 64, 64, 4, ONE),                              # 256 windows
     (256, 1, 64, 64, 8, ONE), (256, 1, 64, 64, 9, 2),      # 512 | 576

@@ -27,7 +27,7 @@ def workspace_bytes(desc, batch):
             + up(2 * desc.n_blocks * desc.n_experts * 64 * 4) + up(desc.n_experts * n * 4))
 
 
-SPLIT_BATCH = 17  # frames of 20x28: 204 windows, two sub-chains of a MoE chain
+SPLIT_BATCH = 22  # frames of 20x28: 264 windows, two sub-chains of a MoE chain
 
 
 @pytest.mark.gpu
