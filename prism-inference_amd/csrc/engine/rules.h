@@ -137,12 +137,14 @@ inline bool chain_attn_w8(const prism_model_desc& d, const ChainPlan& p, int64_t
  * attention a small second round costs less than slower tiles, and the line
  * lies at 5/4 of the grid's tiles per CU: chains with launches of 280 tiles
  * 696 us on 8 waves, 770 on 4; of 296, 745 and 789; of 352, 891 and 855; at
- * the line itself, 320, 816 and 832 on one run, 807 and 789 on another. d128
+ * the line itself, 320, 816 and 832 on one run, 807 and 789 on another; with
+ * more than 32 experts 3/32 further (344: 4 frames of 115x77 819 and 881). d128
  * tiles leave room for two 8-wave workgroups per CU. */
 inline bool expert_w8(int dim, int64_t tiles, int64_t n, int partial, const ChainPlan* p) {
     if (dim != 256) return tiles < 2 * CU_COUNT;
     if (p && p->pair8) return true;
-    return p && p->split > 1 ? tiles <= CU_COUNT * 5 / 4 : (n + 63) / 64 + partial / 2 <= CU_COUNT;
+    const int64_t beside = CU_COUNT * (partial > 32 ? 27 : 25) / 20;
+    return p && p->split > 1 ? tiles <= beside : (n + 63) / 64 + partial / 2 <= CU_COUNT;
 }
 
 /* The leading blocks' expert weights are read past the memory-side cache

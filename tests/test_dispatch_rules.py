@@ -40,6 +40,8 @@ def test_attention_waves(rules):
     (64, 72, 120, 4, 8, 8),       # ... also at 334 tiles
     (64, 66, 118, 4, 8, 8),       # 307 tiles
     (64, 33, 51, 16, 4, 8),       # 275 tiles
+    (64, 115, 77, 4, 4, 8), (64, 75, 75, 6, 4, 8), (64, 45, 80, 10, 4, 4),  # 344, 328 | 352
+    (32, 84, 100, 4, 4, 8), (32, 92, 104, 4, 4, 4),                         # 296 | 336
     (64, 24, 64, 24, 4, 4),       # 576 windows
     (32, 68, 120, 4, 4, 8), (16, 68, 120, 4, 4, 8), (16, 72, 120, 5, 4, 4),
     (64, 24, 64, 23, 8, 8), (64, 96, 120, 3, 4, 4),  # 264 and 288 | 180 and 360: unequal halves
